@@ -70,55 +70,134 @@ struct LaneStack {
     }
 };
 
-// Work fetch of the persistent traversal kernels.  All fetches to one
-// counter serialise across the XCDs, so a queue's ids are split into
-// kFetchSlices contiguous slices with a counter each (kFetchStride words
-// apart).  A wave starts on slice blockIdx.x % kFetchSlices (blocks go to the
-// XCDs in turn, so each XCD starts on its own run of neighbouring rays),
-// reserves kFetchChunk ids at a time and hands them to its idle lanes over
-// several refills; when its slice runs out it moves to the next, and after
-// finding every slice exhausted it has no more work.  Counters only grow,
-// so a slice once exhausted stays so, and every id below n is handed out
-// exactly once.
+// Work fetch of the persistent traversal kernels.  A queue's ids are split
+// into kFetchSlices contiguous slices; a wave belongs to slice blockIdx.x %
+// kFetchSlices (blocks go to the XCDs in turn, so each XCD starts on its own
+// run of neighbouring rays).
+//
+// A wave's first ids are its own by position, without an atomic.  In a queue
+// of at most kFetchChunk ids per wave of the launch every wave owns the even
+// share, at least kFetchMin ids: such queues (late bounces, small frames,
+// small ray batches) take no atomics at all and spread over as many waves as
+// they can, so that few lanes of a wave diverge.  In a larger queue every wave
+// owns one chunk in each of the first `rounds` rounds over its slice, so the
+// waves of an XCD still sweep the slice together.
+// The ids behind the owned ones are handed out dynamically, kFetchChunk at a
+// time, by a counter per slice (kFetchStride words apart): atomics to one
+// counter serialise across the XCDs, at about 11 ns each, and a wave waits for
+// the round trip of its own.  When a slice runs out the wave moves to the
+// next one, looking at its counter before the first addition to it, and after
+// finding every slice exhausted it has no more work.  Counters only grow, so a
+// slice once exhausted stays so, and every id below n is handed out exactly
+// once.
 #ifndef LFH_FETCH_CHUNK
 #define LFH_FETCH_CHUNK 64
 #endif
+#ifndef LFH_FETCH_MIN
+// 1021 rays, 20k triangles: at least 1 / 4 / 16 / 64 rays per wave 71 / 97 / 115 / 110 us (159 us with
+// every wave asking all eight counters); textured 128 x 128 tiles 234 / 239 / 240 / 241 us per pass (738)
+#define LFH_FETCH_MIN 1
+#endif
+#ifndef LFH_FETCH_OWNED
+// eighths of a large queue owned by position: 0 / 4: C0 3.34 / 3.29 ms, 16.8M-ray closest hit 10.32 / 10.23 ms
+// (6: longer when half of the slices hold cheap rays, since owned chunks are never passed on)
+#define LFH_FETCH_OWNED 4
+#endif
 constexpr int kFetchChunk = LFH_FETCH_CHUNK;
+constexpr int kFetchMin = LFH_FETCH_MIN;
+
+// Lane 0's value in a scalar register.
+LFH_DEV unsigned long long wave_first(unsigned long long v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (unsigned long long)hi << 32 | lo;
+}
+// Set bits of `mask` below this lane.
+LFH_DEV int lane_rank(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 struct WaveFetch {
-    unsigned long long base = 0;   // next id of the wave's reservation (same in every lane)
-    int left = 0;                  // ids left in it
-    int slice = -1;                // current slice
-    int tried = 0;                 // slices found exhausted
+    int64_t base = 0;   // next id of the wave's reservation (same in every lane)
+    int64_t own = 0;    // first id of the wave's next owned chunk
+    int left = 0;       // ids left in the reservation
+    int rounds = 0;     // owned chunks not yet taken
+    int slice = 0;      // current slice
+    int tried = 0;      // slices found exhausted
+    int owned = 0;      // ids each wave of the launch owns
+    bool probe = false; // look at the slice's counter before adding to it
+
+    static LFH_HD int waves_of(int s, int blocks, int waves) { return (blocks - s + kFetchSlices - 1) / kFetchSlices * waves; }
+    // blocks x waves: the launch; block, wave: this wave's place in it
+    LFH_DEV void init(int64_t n, int blocks, int waves, int block, int wave) {
+        const int64_t all = (int64_t)blocks * waves;
+        slice = block % kFetchSlices;
+        const int64_t lo = n * slice / kFetchSlices, hi = n * (slice + 1) / kFetchSlices;
+        const int64_t idx = (int64_t)(block / kFetchSlices) * waves + wave;
+        if (n <= all * kFetchChunk) {
+            const int share = (int)((n + all - 1) / all);
+            owned = share < kFetchMin ? kFetchMin : share;
+            base = lo + idx * owned;
+            left = base >= hi ? 0 : (hi - base < owned ? (int)(hi - base) : owned);
+            // equal waves in every slice: nothing is left to fetch
+            if (blocks % kFetchSlices == 0) tried = kFetchSlices;
+        } else {
+            const int64_t r = n / (all * kFetchChunk) * LFH_FETCH_OWNED / 8;
+            rounds = r < 1 ? 1 : (r > (1 << 20) ? 1 << 20 : (int)r);
+            owned = rounds * kFetchChunk;
+            own = lo + idx * kFetchChunk;
+        }
+    }
+    // Nothing owned and nothing to fetch.
+    LFH_DEV bool idle() const { return left == 0 && rounds == 0 && tried == kFetchSlices; }
     // Ids for the lanes in `mask` (nonzero; called by every lane of the wave),
     // in rank order within the mask; n (no work) for lanes left without one.
-    LFH_DEV int64_t next(unsigned long long* ctr, uint64_t mask, int lane, int64_t n, int first_slice) {
+    LFH_DEV int64_t next(unsigned long long* ctr, uint64_t mask, int lane, int64_t n, int blocks, int waves) {
         const int want = __popcll(mask);
-        const int rank = __popcll(mask & ((1ull << lane) - 1ull));
+        const int rank = lane_rank(mask);
         if (left >= want) {
-            const int64_t id = (int64_t)base + rank;
-            base += (unsigned long long)want;
+            const int64_t id = base + rank;
+            base += want;
             left -= want;
             return id;
         }
         const int old = left;
-        int64_t id = rank < old ? (int64_t)base + rank : n;
+        int64_t id = rank < old ? base + rank : n;
         left = 0;
-        if (slice < 0) slice = first_slice;
-        while (tried < kFetchSlices) {
+        while (rounds > 0 || tried < kFetchSlices) {
             const int64_t lo = n * slice / kFetchSlices, hi = n * (slice + 1) / kFetchSlices;
-            unsigned long long nb = 0;
-            if (lane == 0) nb = atomicAdd(ctr + (size_t)slice * kFetchStride, (unsigned long long)kFetchChunk);
-            nb = __shfl(nb, 0);
-            const int64_t start = lo + (int64_t)nb;
-            if (start >= hi) {
-                slice = slice + 1 == kFetchSlices ? 0 : slice + 1;
-                ++tried;
-                continue;
+            int64_t start;
+            if (rounds > 0) {
+                start = own;
+                own += (int64_t)waves_of(slice, blocks, waves) * kFetchChunk;
+                --rounds;
+                if (start >= hi) {
+                    rounds = 0;
+                    continue;
+                }
+            } else {
+                start = lo + (int64_t)waves_of(slice, blocks, waves) * owned;
+                if (start < hi) {
+                    unsigned long long* c = ctr + (size_t)slice * kFetchStride;
+                    unsigned long long nb = 0;
+                    if (lane == 0) {
+                        if (probe) nb = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (start + (int64_t)nb < hi) nb = atomicAdd(c, (unsigned long long)kFetchChunk);
+                    }
+                    start += (int64_t)wave_first(nb);
+                }
+                if (start >= hi) {
+                    slice = slice + 1 == kFetchSlices ? 0 : slice + 1;
+                    ++tried;
+                    probe = true;
+                    continue;
+                }
+                probe = false;
             }
             const int avail = hi - start < kFetchChunk ? (int)(hi - start) : kFetchChunk;
             const int used = want - old < avail ? want - old : avail;
             if (rank >= old && rank < old + used) id = start + (rank - old);
-            base = (unsigned long long)(start + used);
+            base = start + used;
             left = avail - used;
             break;
         }

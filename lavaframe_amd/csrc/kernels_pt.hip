@@ -271,11 +271,13 @@ __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queue(Sh
     float lpdf = 0.f;
     TraceScene ts = sc.tr;
     WaveFetch fetch;
+    fetch.init(n, (int)gridDim.x, kTraceBlock / 64, (int)blockIdx.x, __builtin_amdgcn_readfirstlane(wave));
+    if (fetch.idle()) return;   // wave-uniform; the kernel has no block barrier
     for (;;) {
         const bool need = !active;
         const uint64_t mask = __ballot(need);
         if (mask) {
-            const int64_t id = fetch.next(work, mask, lane, n, (int)(blockIdx.x % kFetchSlices));
+            const int64_t id = fetch.next(work, mask, lane, n, (int)gridDim.x, kTraceBlock / 64);
             if (need) {
                 rid = id;
                 if (rid < n) {

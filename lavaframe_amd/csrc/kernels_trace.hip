@@ -5,6 +5,8 @@
 // work in the same step and takes the next ids of a contiguous chunk its wave
 // reserved with one atomic (WaveFetch), in rank order among the idle lanes, so
 // refills stay coalesced while busy lanes keep traversing.
+#include <algorithm>
+
 #include "dev_trace.h"
 #include "kernels.h"
 
@@ -36,12 +38,14 @@ __global__ __launch_bounds__(kTraceBlock, ANY ? LFH_ANYHIT_WAVES : LFH_TRACE_WAV
     bool active = false;
     int64_t rid = 0;
     WaveFetch fetch;
+    fetch.init(n, (int)gridDim.x, kTraceBlock / 64, (int)blockIdx.x, __builtin_amdgcn_readfirstlane(wave));
+    if (fetch.idle()) return;   // wave-uniform; the kernel has no block barrier
 
     for (;;) {
         const bool need = !active;
         const uint64_t mask = __ballot(need);
         if (mask) {
-            const int64_t id = fetch.next(work, mask, lane, n, (int)(blockIdx.x % kFetchSlices));
+            const int64_t id = fetch.next(work, mask, lane, n, (int)gridDim.x, kTraceBlock / 64);
             if (need) {
                 rid = id;
                 if (rid < n) {
@@ -119,7 +123,10 @@ hipError_t lfh_launch_trace(const TraceLaunch& L, hipStream_t stream) {
     // L.grid_blocks sizes the spill buffer; each variant launches at most its own resident count
     const int* v = variant_blocks();
     const int which = L.any ? 1 : (L.counts ? 2 : 0);
-    const int blocks = v[which] < L.grid_blocks ? v[which] : L.grid_blocks;
+    const int resident = v[which] < L.grid_blocks ? v[which] : L.grid_blocks;
+    // small batches: a wave for every kFetchMin rays, in equal numbers on all slices
+    const int64_t few = (L.n + kFetchMin * (kTraceBlock / 64) - 1) / (kFetchMin * (kTraceBlock / 64));
+    const int blocks = (int)std::min<int64_t>(resident, (few + kFetchSlices - 1) / kFetchSlices * kFetchSlices);
     hipLaunchKernelGGL(k_zero_fetch, dim3(1), dim3(64), 0, stream, L.work);
     if (L.any) {
         hipLaunchKernelGGL((k_trace<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, L.scene, L.rays, L.n,
