@@ -22,10 +22,14 @@ constexpr float kTwoPi = 6.28318530717958648f;
 //   internal node : index (< 2^30)
 //   BLAS leaf     : 0x80000000 | (count << 28) | first triangle slot (< 2^28)
 //   TLAS leaf     : 0x40000000 | instance index (< 2^30)
-//   sentinel      : 0xFFFFFFFF (stack bottom / return from a BLAS)
+//   sentinel      : 0xFFFFFFFF (absent child; end marker of the stack)
+//   return marker : 0xFFFFFFFE (on the stack below a BLAS; no leaf has this ref:
+//                   7 triangles from slot 2^28 - 2)
 constexpr uint32_t kRefSentinel = 0xFFFFFFFFu;
+constexpr uint32_t kRefReturn = 0xFFFFFFFEu;
 constexpr uint32_t kRefLeafBit = 0x80000000u;
 constexpr uint32_t kRefInstBit = 0x40000000u;
+LFH_HD bool ref_is_node(uint32_t r) { return r < kRefInstBit; }
 LFH_HD bool ref_is_leaf(uint32_t r) { return (r & kRefLeafBit) != 0; }
 LFH_HD bool ref_is_inst(uint32_t r) { return (r & 0xC0000000u) == kRefInstBit; }
 LFH_HD uint32_t leaf_first(uint32_t r) { return r & 0x0FFFFFFFu; }
@@ -38,7 +42,8 @@ LFH_HD uint32_t make_inst(uint32_t inst) { return kRefInstBit | inst; }
 // as structure of arrays, child k in lane k of each float4:
 //   f4[0..2] = min.x, min.y, min.z    f4[3..5] = max.x, max.y, max.z
 //   f4[6]    = as_float(child refs)   f4[7]    = 0
-//   an absent child has ref kRefSentinel.
+//   an absent child has ref kRefSentinel and the empty box (+inf, -inf), which
+//   no ray with finite nonzero inv enters.
 // (Host intermediate: the BVH2 node of 64 B with both child boxes,
 //  (lmin, lmax, rmin, rmax, left ref, right ref), collapsed into BVH4 nodes.)
 // Triangle, 48 B, in vert_indices slot order:
@@ -47,32 +52,19 @@ LFH_HD uint32_t make_inst(uint32_t inst) { return kRefInstBit | inst; }
 // Instance, 64 B: rows 0..2 of inverse(M) as (inv[0][r], inv[1][r], inv[2][r],
 //   inv[3][r]) and (as_float(blas ref), as_float(material), as_float(index), 0).
 
-// Traversal stack: the newest kLdsStack entries of a lane live in LDS, older
-// ones spill to a per-lane global area of kSpillStride entries.
+// Traversal stack: the first kLdsStack entries of a lane live in LDS, deeper
+// ones in a per-lane global area of kSpillStride entries.
 #ifndef LFH_LDS_STACK
-#define LFH_LDS_STACK 16
+#define LFH_LDS_STACK 16   // 24 entries: any hit 2207 against 2116 us (8.4M incoherent rays), closest hit the same
 #endif
 #ifndef LFH_TRACE_WAVES
-// Waves per SIMD the ray-batch traversal kernel is register-budgeted for,
-// closest hit and any hit.  With the octant slab (packed offsets), 1M-triangle
-// soup: closest 6 waves 1641 Mrays/s (incoherent 1015, 28 B/lane spilled),
-// 5 waves 1649 (incoherent 1038, coherent 3528 against 3672); any hit 6 waves
-// 3876, 5 waves 3649.
+// Waves per SIMD the ray-batch closest-hit kernel is register-budgeted for (87 VGPRs, no
+// spills).  16.8M rays, 1M-triangle soup: 5 waves 6.22 ms, 6 waves 6.23 ms.
 #define LFH_TRACE_WAVES 5
 #endif
-#ifndef LFH_SLAB_OCTANT
-#define LFH_SLAB_OCTANT 1   // node box tests with the near / far planes picked by the ray octant: C1 1633 / 1590 Mrays/s (incoherent 1011 / 984), any hit 3863 / 3701, C2 398 / 392 Msamples/s
-#endif
 #ifndef LFH_ANYHIT_WAVES
-// any hit with 16-step slices: 5 / 6 / 7 / 8 waves per SIMD 4084 / 4305 / 4203 / 3860 Mrays/s
-// (7 and 8 spill 28 and 56 B per lane); closest hit at 6 waves 1642.5 against 1649 at 5
+// the same for any hit (79 VGPRs): 5 and 6 waves 0.794 ms for 2.1M rays
 #define LFH_ANYHIT_WAVES 6
-#endif
-#ifndef LFH_OCTANT_PACKED
-#define LFH_OCTANT_PACKED 1   // the three near-plane offsets and the flag in one register (0: three + a flag)
-#endif
-#ifndef LFH_POP_CULL
-#define LFH_POP_CULL 0   // 1: keep box entry distances on the stack and drop stale entries at pop
 #endif
 // Work counters of the persistent traversal kernels: a queue's ray ids are
 // split into kFetchSlices contiguous slices, each with its own counter
@@ -88,18 +80,19 @@ constexpr int kFetchWords = kFetchSlices * kFetchStride;
 constexpr int kWorkTotals = 2 * kFetchWords;
 constexpr int kWorkWords = kWorkTotals + 8;
 #ifndef LFH_TRACE_SLICE
-#define LFH_TRACE_SLICE 32   // C1 / C0 / C2: 16: 1557 / 1195 / 326, 24: 1557 / 1226 / 329, 32: 1573 / 1235 / 328, 48: 1558 / 1224 / 317, 96: 1457 / 1233 / 295
+// 16 / 24 / 32 / 48 steps: 16.8M closest hits 5.90 / 5.92 / 5.92 / 6.09 ms, instanced 1080p frame
+// 22.0 / 22.1 / 22.3 / 22.6 ms, C0 3.14 / 3.10 / 3.10 / 3.09 ms, served mix 5.04 / 4.93 / 4.98 / 4.94 ms
+#define LFH_TRACE_SLICE 24
 #endif
 constexpr int kTraceSlice = LFH_TRACE_SLICE;  // traversal steps between refills of a wave's idle lanes
 #ifndef LFH_ANY_SLICE
-// the same for any-hit queries (C1 any hit; shadow rays of the path tracer): 32 steps 3885-3893
-// Mrays/s, 24: 4107-4131, 16: 4288-4296, 12: 4293, 8: 4257 (C2 421.5 against 428 at 12-24)
+// the same for any-hit queries: 8 / 12 / 16 / 24 / 32 steps 1003 / 798 / 794 / 797 / 989 us for 2.1M rays
 #define LFH_ANY_SLICE 16
 #endif
 constexpr int kAnySlice = LFH_ANY_SLICE;
-constexpr int kLdsStack = LFH_LDS_STACK;  // LDS entries per lane (power of 2)
+constexpr int kLdsStack = LFH_LDS_STACK;  // LDS entries per lane
 constexpr int kTraceBlock = 256;        // threads per traversal block (4 wave64)
-constexpr uint32_t kSpillStride = 128;  // max stack entries per lane
+constexpr uint32_t kSpillStride = 128;  // global entries per lane; the most a scene's traversal may need
 
 struct TraceScene {
     const float4* nodes;
@@ -141,29 +134,46 @@ LFH_DEV float as_f(uint32_t u) { return __uint_as_float(u); }
 LFH_DEV uint32_t as_u(float f) { return __float_as_uint(f); }
 
 // ---- slab test (intersection.glsl:56-72) -------------------------------------
-// Returns the reference's AABBIntersect value: t0 if the box is hit in front
-// (t0 > 0), the exit t1 if the origin is inside, -1 on a miss.  `entry`
-// receives max(t0, 0) for culling.  min/max are IEEE minNum/maxNum.
-// slab() with the near and far plane of each axis already chosen by the
-// ray's octant (finite inv): the same t0 / t1, bit for bit, without the
-// per-axis min / max.
-LFH_DEV float slab_octant(V3 bnear, V3 bfar, V3 o, V3 inv, float* entry) {
-    const float nx = (bnear.x - o.x) * inv.x, ny = (bnear.y - o.y) * inv.y, nz = (bnear.z - o.z) * inv.z;
-    const float fx = (bfar.x - o.x) * inv.x, fy = (bfar.y - o.y) * inv.y, fz = (bfar.z - o.z) * inv.z;
-    const float t1 = fminf(fx, fminf(fy, fz));
+// Order key of a box the ray enters in front of its origin (AABBIntersect > 0)
+// at a distance t0 <= lim, infinity for any other box.  min/max are IEEE
+// minNum/maxNum.  Both lower limits go into max(t0, the least positive float),
+// for closest hit both upper ones into min(t1, lim), so one comparison
+// decides (two for any hit).
+//
+// The key decides how many nodes a ray visits, not what it hits:
+//   closest hit  t0, also where it is negative: of the boxes around the origin
+//                the one reaching furthest back goes first.  Ordering those by
+//                their exit t1 (AABBIntersect's value) costs an incoherent ray
+//                twice the visits: 8.4M rays 9.01 ms against 3.81 ms, and 3.85 ms
+//                with all of them at key 0.
+//   any hit      the longest stretch inside the box first, where a hit is
+//                likeliest: 8.4M rays 2.20 ms against 3.13 ms by t0, 2.79 ms by
+//                AABBIntersect's value, 3.47 ms by t1, 2.53 ms by -t1.
+constexpr float kLeastPositive = 1.401298464e-45f;
+template <bool ANY>
+LFH_DEV float slab_entry(float nx, float ny, float nz, float fx, float fy, float fz, float lim) {
     const float t0 = fmaxf(nx, fmaxf(ny, nz));
-    *entry = t0;
-    return (t1 >= t0) ? (t0 > 0.f ? t0 : t1) : -1.0f;
+    const float none = __builtin_inff();
+    if (ANY) {
+        const float c0 = fmaxf(t0, kLeastPositive);
+        const float t1 = fminf(fx, fminf(fy, fz));
+        return t1 >= c0 && c0 <= lim ? c0 - t1 : none;
+    }
+    const float t1 = fminf(fx, fminf(fy, fminf(fz, lim)));
+    return t1 >= fmaxf(t0, kLeastPositive) ? t0 : none;
 }
-LFH_DEV float slab(V3 bmin, V3 bmax, V3 o, V3 inv, float* entry) {
-    float fx = (bmax.x - o.x) * inv.x, fy = (bmax.y - o.y) * inv.y, fz = (bmax.z - o.z) * inv.z;
-    float nx = (bmin.x - o.x) * inv.x, ny = (bmin.y - o.y) * inv.y, nz = (bmin.z - o.z) * inv.z;
-    float tmaxx = fmaxf(fx, nx), tmaxy = fmaxf(fy, ny), tmaxz = fmaxf(fz, nz);
-    float tminx = fminf(fx, nx), tminy = fminf(fy, ny), tminz = fminf(fz, nz);
-    float t1 = fminf(tmaxx, fminf(tmaxy, tmaxz));
-    float t0 = fmaxf(tminx, fmaxf(tminy, tminz));
-    *entry = t0;
-    return (t1 >= t0) ? (t0 > 0.f ? t0 : t1) : -1.0f;
+// The near and far plane of each axis already chosen by the ray's octant
+// (finite inv): the same t0 / t1, bit for bit, without the per-axis min / max.
+template <bool ANY>
+LFH_DEV float slab_octant(V3 bnear, V3 bfar, V3 o, V3 inv, float lim) {
+    return slab_entry<ANY>((bnear.x - o.x) * inv.x, (bnear.y - o.y) * inv.y, (bnear.z - o.z) * inv.z,
+                      (bfar.x - o.x) * inv.x, (bfar.y - o.y) * inv.y, (bfar.z - o.z) * inv.z, lim);
+}
+template <bool ANY>
+LFH_DEV float slab(V3 bmin, V3 bmax, V3 o, V3 inv, float lim) {
+    const float fx = (bmax.x - o.x) * inv.x, fy = (bmax.y - o.y) * inv.y, fz = (bmax.z - o.z) * inv.z;
+    const float nx = (bmin.x - o.x) * inv.x, ny = (bmin.y - o.y) * inv.y, nz = (bmin.z - o.z) * inv.z;
+    return slab_entry<ANY>(fminf(fx, nx), fminf(fy, ny), fminf(fz, nz), fmaxf(fx, nx), fmaxf(fy, ny), fmaxf(fz, nz), lim);
 }
 
 // ---- Moller-Trumbore as written in closest_hit.glsl:119-134 ------------------

@@ -17,56 +17,41 @@
 //   * exact-t ties between triangles go to the lowest (instance, prim) pair
 //     instead of the first one found, so the answer does not depend on visit
 //     order;
-//   * the per-lane stack keeps its newest entries in LDS (kLdsStack of them)
-//     with their box entry distances, and spills older ones to a per-lane
-//     global area; a popped entry whose entry distance is beyond the current
-//     best t (times `cull`) is skipped.
+//   * the per-lane stack keeps its first kLdsStack entries in LDS and deeper
+//     ones in a per-lane global area.
 #pragma once
 #include "dev_common.h"
 
 namespace lfhd {
 
 
+// Entry e of a lane's stack is in LDS for e < kLdsStack (at lds[e * 64]) and in
+// the lane's global area above that.  Entry 0 is the end marker kRefSentinel.
+// The address spaces are part of the types: a pop that selects between two
+// generic pointers becomes one flat load, which waits for both memories.
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+typedef __attribute__((address_space(1))) uint32_t GlobalWord;
 struct LaneStack {
-    uint32_t* lds;    // this lane's column of refs: entry e at lds[e * 64]
-    float* ldk;       // entry distances of the LDS entries, same indexing
-    uint32_t* spill;  // this lane's global spill area (refs only)
-    int sp, lo;
+    LdsWord* lds;       // this lane's LDS column
+    GlobalWord* spill;  // this lane's global area
+    int sp;           // entries
     bool overflow;
-    LFH_DEV void reset() { sp = 0; lo = 0; overflow = false; }
-    LFH_DEV void push(uint32_t v, float key) {
-        if (sp - lo == kLdsStack) {
-            spill[lo] = lds[(lo & (kLdsStack - 1)) * 64];
-            lo++;
-        }
-        if (sp >= (int)kSpillStride) { overflow = true; return; }
-        lds[(sp & (kLdsStack - 1)) * 64] = v;
-        if (LFH_POP_CULL) ldk[(sp & (kLdsStack - 1)) * 64] = key;
+    LFH_DEV void reset() {
+        lds[0] = kRefSentinel;
+        sp = 1;
+        overflow = false;
+    }
+    LFH_DEV void push(uint32_t v) {
+        if (sp < kLdsStack) lds[sp * 64] = v;
+        else if (sp < kLdsStack + (int)kSpillStride) spill[sp - kLdsStack] = v;
+        else { overflow = true; return; }
         sp++;
     }
-    // Pops the newest entry; entries that come back from the spill area have
-    // lost their distance and are never culled.
-    LFH_DEV uint32_t pop(float& key) {
-        if (sp <= 0) {
-            key = -kInfinity;
-            return kRefSentinel;
-        }
+    LFH_DEV uint32_t pop() {
         sp--;
-        if (sp < lo) {
-            lo = sp;
-            key = -kInfinity;
-            return spill[sp];
-        }
-        key = LFH_POP_CULL ? ldk[(sp & (kLdsStack - 1)) * 64] : -kInfinity;
-        return lds[(sp & (kLdsStack - 1)) * 64];
-    }
-    // Pops until an entry whose box entry distance is within lim (or a marker).
-    LFH_DEV uint32_t pop_live(float lim) {
-        for (;;) {
-            float k;
-            const uint32_t r = pop(k);
-            if (r == kRefSentinel || k <= lim) return r;
-        }
+        uint32_t r = lds[(sp < kLdsStack ? sp : 0) * 64];
+        if (__builtin_expect(sp >= kLdsStack, 0)) r = spill[sp - kLdsStack];
+        return r;
     }
 };
 
@@ -216,53 +201,32 @@ struct TraceState {
     V3 o, d, inv;       // current-space ray
     float tmin, tbest;
     uint32_t cur;
-    bool inBlas;
     int curInst, curMat;
     int bestPrim, bestInst, bestMat, bestSlot;
     float bu, bv;
     bool occluded;
-#if LFH_SLAB_OCTANT
-#if LFH_OCTANT_PACKED
-    uint32_t oct;   // near-plane byte offsets x | y << 8 | z << 16, bit 24: inv has an infinite component
-#else
-    uint32_t nearx, neary, nearz;   // byte offsets of the near-side box planes in a node (ray octant)
-    bool inf_inv;                   // some component of inv is infinite (axis-parallel ray)
-#endif
-#endif
+    uint32_t oct;   // near-plane byte offsets x | y << 8 | z << 16, bit 24: inv has an infinite or zero component
 };
 
-#if LFH_SLAB_OCTANT
 // The near-side plane of each axis follows from the sign of inv: min at
 // bytes 0/16/32 of a node, max at 48/64/80.  For finite inv the near plane's
 // distance equals the per-axis min of the two (t = (b - o) inv is monotonic
 // in b), bit for bit; an infinite component (d = +-0) can make one of them
 // 0 * inf = NaN, which the min/max form resolves differently, so such rays
-// take the min/max form.
+// take the min/max form (and so do rays with a zero component of inv, whose
+// distances to the infinite planes of an absent child would be NaN).
 LFH_DEV void set_octant(TraceState& s) {
     const uint32_t nx = signbit(s.inv.x) ? 48u : 0u, ny = signbit(s.inv.y) ? 64u : 16u,
                    nz = signbit(s.inv.z) ? 80u : 32u;
-    const bool inf = !(isfinite(s.inv.x) && isfinite(s.inv.y) && isfinite(s.inv.z));
-#if LFH_OCTANT_PACKED
+    const float big = fmaxf(fmaxf(fabsf(s.inv.x), fabsf(s.inv.y)), fabsf(s.inv.z));
+    const float small = fminf(fminf(fabsf(s.inv.x), fabsf(s.inv.y)), fabsf(s.inv.z));
+    const bool inf = !(big < __builtin_inff() && small > 0.0f);
     s.oct = nx | (ny << 8) | (nz << 16) | (inf ? 1u << 24 : 0u);
-#else
-    s.nearx = nx;
-    s.neary = ny;
-    s.nearz = nz;
-    s.inf_inv = inf;
-#endif
 }
-#if LFH_OCTANT_PACKED
 LFH_DEV bool octant_inf(const TraceState& s) { return (s.oct >> 24) != 0; }
 LFH_DEV uint32_t near_x(const TraceState& s) { return s.oct & 0xFFu; }
 LFH_DEV uint32_t near_y(const TraceState& s) { return (s.oct >> 8) & 0xFFu; }
 LFH_DEV uint32_t near_z(const TraceState& s) { return (s.oct >> 16) & 0xFFu; }
-#else
-LFH_DEV bool octant_inf(const TraceState& s) { return s.inf_inv; }
-LFH_DEV uint32_t near_x(const TraceState& s) { return s.nearx; }
-LFH_DEV uint32_t near_y(const TraceState& s) { return s.neary; }
-LFH_DEV uint32_t near_z(const TraceState& s) { return s.nearz; }
-#endif
-#endif
 
 LFH_DEV void trace_init(TraceState& s, LaneStack& st, V3 O, V3 D, float tmin, float tmax, uint32_t root) {
     s.O = O;
@@ -274,7 +238,6 @@ LFH_DEV void trace_init(TraceState& s, LaneStack& st, V3 O, V3 D, float tmin, fl
     s.tmin = tmin;
     s.tbest = tmax;
     s.cur = root;
-    s.inBlas = false;
     s.curInst = -1;
     s.curMat = 0;
     s.bestPrim = -1;
@@ -284,9 +247,7 @@ LFH_DEV void trace_init(TraceState& s, LaneStack& st, V3 O, V3 D, float tmin, fl
     s.bu = 0.f;
     s.bv = 0.f;
     s.occluded = false;
-#if LFH_SLAB_OCTANT
     set_octant(s);
-#endif
     st.reset();
 }
 
@@ -335,109 +296,126 @@ LFH_DEV void enter_instance(const TraceScene& sc, TraceState& s, LaneStack& st, 
     s.o = xform_inv(r0, r1, r2, s.O, 1.0f);
     s.d = xform_inv(r0, r1, r2, s.D, 0.0f);
     s.inv = rcp3(s.d);
-#if LFH_SLAB_OCTANT
     set_octant(s);
-#endif
-    st.push(kRefSentinel, -kInfinity);
-    s.inBlas = true;
+    st.push(kRefReturn);
     s.curInst = (int)inst;
     s.curMat = (int)as_u(meta.y);
     s.cur = as_u(meta.x);
 }
 
-// BVH4 node: slab-test the four child boxes, descend into the nearest hit
-// child, push the others farthest first.
-template <bool STATS>
-LFH_DEV void visit_node(const TraceScene& sc, TraceState& s, LaneStack& st, uint32_t cur, float cull,
-                        TraceStats* stats) {
+// A node's near planes (a, b, c), far planes (d, e, f) and child refs.
+struct NodeRec {
+    float4 a, b, c, d, e, f, rf;
+};
+// near and far planes read by per-lane offsets: the per-axis min/max drop out
+LFH_DEV void load_node(const TraceScene& sc, const TraceState& s, uint32_t cur, NodeRec& n) {
+    const char* nb = reinterpret_cast<const char*>(sc.nodes);
+    const uint32_t off = cur * 128u;
+    const uint32_t ox = near_x(s), oy = near_y(s), oz = near_z(s);
+    n.a = *reinterpret_cast<const float4*>(nb + (off + ox));
+    n.b = *reinterpret_cast<const float4*>(nb + (off + oy));
+    n.c = *reinterpret_cast<const float4*>(nb + (off + oz));
+    n.d = *reinterpret_cast<const float4*>(nb + (off + (48u - ox)));
+    n.e = *reinterpret_cast<const float4*>(nb + (off + (80u - oy)));
+    n.f = *reinterpret_cast<const float4*>(nb + (off + (112u - oz)));
+    n.rf = *reinterpret_cast<const float4*>(nb + (off + 96u));
+}
+
+// BVH4 node: slab-test the four child boxes, push the hit children last in
+// order first.  Returns the first one, or kRefSentinel when none is hit.
+//
+// Bound by VALU issue (77 % busy on 16.8M mixed rays, 40 % of the lanes active
+// on average): the test is 17 instructions per child, the sort 25, the pushes
+// 12 without a branch per child.  With one pop per step for all lanes and the
+// order keys of slab_entry the 1M-triangle soup's closest hit went from 1650 to
+// 2840 Mrays/s (incoherent half 1037 -> 2380), any hit from 3270 to 3960.
+// Loading the nodes of a step before its leaf tests, to overlap the two
+// latencies, spills (6.24 against 5.95 ms; any hit 6.9 against 2.2 ms).
+template <bool ANY, bool STATS>
+LFH_DEV uint32_t visit_node(const NodeRec& nd, bool plain, TraceState& s, LaneStack& st, float cull,
+                            TraceStats* stats) {
     if (STATS) stats->nint++;
     const float lim = s.tbest * cull;
-    float h[4], e[4];
-    uint32_t r[4];
-#if LFH_SLAB_OCTANT
-    if (__ballot(octant_inf(s)) == 0) {   // wave-uniform
-        // near and far planes read by per-lane offsets: the per-axis min/max drop out
-        const char* nb = reinterpret_cast<const char*>(sc.nodes);
-        const uint32_t off = cur * 128u;
-        const uint32_t ox = near_x(s), oy = near_y(s), oz = near_z(s);
-        const float4 nx = *reinterpret_cast<const float4*>(nb + (off + ox));
-        const float4 ny = *reinterpret_cast<const float4*>(nb + (off + oy));
-        const float4 nz = *reinterpret_cast<const float4*>(nb + (off + oz));
-        const float4 fx = *reinterpret_cast<const float4*>(nb + (off + (48u - ox)));
-        const float4 fy = *reinterpret_cast<const float4*>(nb + (off + (80u - oy)));
-        const float4 fz = *reinterpret_cast<const float4*>(nb + (off + (112u - oz)));
-        const float4 rf = *reinterpret_cast<const float4*>(nb + (off + 96u));
-        r[0] = as_u(rf.x); r[1] = as_u(rf.y); r[2] = as_u(rf.z); r[3] = as_u(rf.w);
-        h[0] = slab_octant(v3(nx.x, ny.x, nz.x), v3(fx.x, fy.x, fz.x), s.o, s.inv, &e[0]);
-        h[1] = slab_octant(v3(nx.y, ny.y, nz.y), v3(fx.y, fy.y, fz.y), s.o, s.inv, &e[1]);
-        h[2] = slab_octant(v3(nx.z, ny.z, nz.z), v3(fx.z, fy.z, fz.z), s.o, s.inv, &e[2]);
-        h[3] = slab_octant(v3(nx.w, ny.w, nz.w), v3(fx.w, fy.w, fz.w), s.o, s.inv, &e[3]);
-    } else
-#endif
-    {
-        const float4* np = sc.nodes + (size_t)cur * 8;
-        const float4 mnx = np[0], mny = np[1], mnz = np[2], mxx = np[3], mxy = np[4], mxz = np[5];
-        const float4 rf = np[6];
-        r[0] = as_u(rf.x); r[1] = as_u(rf.y); r[2] = as_u(rf.z); r[3] = as_u(rf.w);
-        h[0] = slab(v3(mnx.x, mny.x, mnz.x), v3(mxx.x, mxy.x, mxz.x), s.o, s.inv, &e[0]);
-        h[1] = slab(v3(mnx.y, mny.y, mnz.y), v3(mxx.y, mxy.y, mxz.y), s.o, s.inv, &e[1]);
-        h[2] = slab(v3(mnx.z, mny.z, mnz.z), v3(mxx.z, mxy.z, mxz.z), s.o, s.inv, &e[2]);
-        h[3] = slab(v3(mnx.w, mny.w, mnz.w), v3(mxx.w, mxy.w, mxz.w), s.o, s.inv, &e[3]);
-    }
-    int nv = 0;
+    const float none = __builtin_inff();
+    float h[4];      // order key of a hit child, infinity otherwise
+    uint32_t r[4] = {as_u(nd.rf.x), as_u(nd.rf.y), as_u(nd.rf.z), as_u(nd.rf.w)};
+    const float4 nx = nd.a, ny = nd.b, nz = nd.c, fx = nd.d, fy = nd.e, fz = nd.f;
+    if (plain) {
+        h[0] = slab_octant<ANY>(v3(nx.x, ny.x, nz.x), v3(fx.x, fy.x, fz.x), s.o, s.inv, lim);
+        h[1] = slab_octant<ANY>(v3(nx.y, ny.y, nz.y), v3(fx.y, fy.y, fz.y), s.o, s.inv, lim);
+        h[2] = slab_octant<ANY>(v3(nx.z, ny.z, nz.z), v3(fx.z, fy.z, fz.z), s.o, s.inv, lim);
+        h[3] = slab_octant<ANY>(v3(nx.w, ny.w, nz.w), v3(fx.w, fy.w, fz.w), s.o, s.inv, lim);
+    } else {
+        h[0] = slab<ANY>(v3(nx.x, ny.x, nz.x), v3(fx.x, fy.x, fz.x), s.o, s.inv, lim);
+        h[1] = slab<ANY>(v3(nx.y, ny.y, nz.y), v3(fx.y, fy.y, fz.y), s.o, s.inv, lim);
+        h[2] = slab<ANY>(v3(nx.z, ny.z, nz.z), v3(fx.z, fy.z, fz.z), s.o, s.inv, lim);
+        h[3] = slab<ANY>(v3(nx.w, ny.w, nz.w), v3(fx.w, fy.w, fz.w), s.o, s.inv, lim);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const bool ok = r[k] != kRefSentinel && h[k] > 0.f && e[k] <= lim;
-        nv += ok ? 1 : 0;
-        h[k] = ok ? fminf(h[k], 3.0e38f) : __builtin_inff();
+        for (int k = 0; k < 4; ++k)
+            if (r[k] == kRefSentinel) h[k] = none;
     }
-    // sort by hit distance (absent / culled children last)
+    // first in order first, absent / culled children last
 #define LFH_CSWAP(a, b)                                              \
-    if (h[b] < h[a]) {                                               \
-        float th = h[a]; h[a] = h[b]; h[b] = th;                     \
-        float te = e[a]; e[a] = e[b]; e[b] = te;                     \
-        uint32_t tr = r[a]; r[a] = r[b]; r[b] = tr;                  \
+    {                                                                \
+        const bool sw = h[b] < h[a];                                 \
+        const float lo = sw ? h[b] : h[a], hi = sw ? h[a] : h[b];    \
+        const uint32_t rl = sw ? r[b] : r[a], rh = sw ? r[a] : r[b]; \
+        h[a] = lo; h[b] = hi;                                        \
+        r[a] = rl; r[b] = rh;                                        \
     }
     LFH_CSWAP(0, 1) LFH_CSWAP(2, 3) LFH_CSWAP(0, 2) LFH_CSWAP(1, 3) LFH_CSWAP(1, 2)
 #undef LFH_CSWAP
-    if (nv == 0) {
-        s.cur = st.pop_live(lim);
+    if (__builtin_expect(st.sp <= kLdsStack - 3, 1)) {
+        // room for three: each write lands on the slot the last valid one left
+        LdsWord* p = st.lds + st.sp * 64;
+        int n = 0;
+        p[0] = r[3];
+        n += h[3] < none ? 64 : 0;
+        p[n] = r[2];
+        n += h[2] < none ? 64 : 0;
+        p[n] = r[1];
+        n += h[1] < none ? 64 : 0;
+        st.sp += n / 64;
     } else {
-        if (nv > 3) st.push(r[3], e[3]);
-        if (nv > 2) st.push(r[2], e[2]);
-        if (nv > 1) st.push(r[1], e[1]);
-        s.cur = r[0];
+        if (h[3] < none) st.push(r[3]);
+        if (h[2] < none) st.push(r[2]);
+        if (h[1] < none) st.push(r[1]);
     }
+    return h[0] < none ? r[0] : kRefSentinel;
 }
 
 // Runs up to `budget` loop steps; returns true when the traversal finished.
+// A step is a node visit, a leaf or an instance entry, then one pop for all
+// the lanes that have nothing left below.
 template <bool ANY, bool STATS>
 LFH_DEV bool trace_run(const TraceScene& sc, TraceState& s, LaneStack& st, float cull, int budget,
                        TraceStats* stats) {
+    if (s.cur == kRefSentinel) return true;
     for (int it = 0; it < budget; ++it) {
-        uint32_t cur = s.cur;
-        if (cur == kRefSentinel) {
-            if (s.inBlas) {
-                s.inBlas = false;
+        const uint32_t cur = s.cur;
+        uint32_t next = kRefSentinel;
+        if (ref_is_node(cur)) {
+            NodeRec nd;
+            load_node(sc, s, cur, nd);
+            next = visit_node<ANY, STATS>(nd, __ballot(octant_inf(s)) == 0, s, st, cull, stats);
+        } else if (ref_is_leaf(cur)) {
+            if (leaf_test<ANY, STATS>(sc, s, cur, stats)) return true;
+        } else {
+            enter_instance<STATS>(sc, s, st, cur, stats);
+            next = s.cur;
+        }
+        if (next == kRefSentinel) {
+            next = st.pop();
+            if (next == kRefReturn) {
                 s.o = s.O;
                 s.d = s.D;
                 s.inv = s.invD;
-#if LFH_SLAB_OCTANT
                 set_octant(s);
-#endif
-                s.cur = st.pop_live(s.tbest * cull);
-                continue;
+                next = st.pop();
             }
-            return true;
+            if (next == kRefSentinel) return true;
         }
-        if (ref_is_leaf(cur)) {
-            if (leaf_test<ANY, STATS>(sc, s, cur, stats)) return true;
-            s.cur = st.pop_live(s.tbest * cull);
-        } else if (ref_is_inst(cur)) {
-            enter_instance<STATS>(sc, s, st, cur, stats);
-        } else {
-            visit_node<STATS>(sc, s, st, cur, cull, stats);
-        }
+        s.cur = next;
         if (st.overflow) return true;
     }
     return false;

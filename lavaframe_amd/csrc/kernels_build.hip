@@ -412,7 +412,8 @@ __global__ __launch_bounds__(kBlk) void k_level_write(CollapseArgs a, Level q, i
     float row[8][4];
     for (int k = 0; k < 4; ++k) {
         uint32_t ref = kRefSentinel;
-        float4 lo = make_float4(1.f, 1.f, 1.f, 0.f), hi = make_float4(-1.f, -1.f, -1.f, 0.f);
+        const float none = __builtin_inff();   // box of an absent child
+        float4 lo = make_float4(none, none, none, 0.f), hi = make_float4(-none, -none, -none, 0.f);
         if (k < c) {
             const int n = ch[k];
             // exact vertex bounds, as the reference builder boxes primitives: a

@@ -244,7 +244,7 @@ LFH_DEV bool light_any(const ShadeScene& sc, V3 o, V3 d, float maxDist) {
 
 template <bool SHADOW, bool MULTI>
 #ifndef LFH_QUEUE_WAVES
-#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD; with the octant slab 6: C0 1206 / C2 396 Msamples/s, 5: 1223 / 379 (C3 pass cost equal)
+#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD: 6 / 5: C0 3.10 / 3.26 ms, instanced 1080p frame 22.3 / 24.4 ms
 #endif
 __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queue(ShadeScene sc, const JobDev* __restrict__ jobs,
                                                              const float4* __restrict__ q,
@@ -254,14 +254,12 @@ __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queue(Sh
                                                              unsigned long long* __restrict__ work, float cull,
                                                              int* __restrict__ err) {
     __shared__ uint32_t stk[kTraceBlock / 64][kLdsStack][64];
-    __shared__ float stkd[kTraceBlock / 64][LFH_POP_CULL ? kLdsStack : 1][64];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     LaneStack st;
-    st.lds = &stk[wave][0][lane];
-    st.ldk = &stkd[wave][0][lane];
-    st.spill = spill + gtid * kSpillStride;
+    st.lds = (LdsWord*)&stk[wave][0][lane];
+    st.spill = (GlobalWord*)(spill + gtid * kSpillStride);
     st.reset();
     const int64_t n = (int64_t)*count;
     TraceState s;

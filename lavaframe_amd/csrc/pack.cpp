@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <unordered_map>
 #include <string>
 #include <vector>
@@ -402,7 +403,7 @@ struct Widen {
             out.resize(out.size() + 32, 0.0f);
             float* o = &out[idx * 32];
             for (uint32_t k = 0; k < 4; ++k) {
-                float b[6] = {1.f, 1.f, 1.f, -1.f, -1.f, -1.f};
+                float b[6] = {kEmpty, kEmpty, kEmpty, -kEmpty, -kEmpty, -kEmpty};
                 uint32_t ref = lfhd::kRefSentinel;
                 if (k < cnt) {
                     tri_box(first + k, b);
@@ -475,7 +476,7 @@ struct Widen {
         float* o = &out[idx * 32];
         for (int k = 0; k < 4; ++k) {
             const float* b = k < n ? ch[k].box : nullptr;
-            for (int a = 0; a < 6; ++a) o[a * 4 + k] = b ? b[a] : (a < 3 ? 1.0f : -1.0f);
+            for (int a = 0; a < 6; ++a) o[a * 4 + k] = b ? b[a] : (a < 3 ? kEmpty : -kEmpty);
             std::memcpy(&o[24 + k], &refs[k], 4);
         }
         *need = (n - 1) + worst;
@@ -494,6 +495,7 @@ struct Widen {
     // children keeps each child's exact box from the BVH2 tree (or the
     // triangle's vertex box inside its leaf's box), so the triangles a ray
     // tests are among those the BVH2 traversal tests.
+    static constexpr float kEmpty = std::numeric_limits<float>::infinity();   // box of an absent child: (+inf, -inf)
     static constexpr float kCostNode = 1.0f;
     static constexpr float kCostTri = LFH_WIDEN_TRI_COST;
     static constexpr float kCostInst = 0.5f;

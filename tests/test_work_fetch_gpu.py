@@ -34,3 +34,44 @@ def test_every_ray_of_a_batch_is_traced_once(world, n):
     for f in ("t", "u", "v"):
         assert np.array_equal(got[f].view(np.uint32), want[f].view(np.uint32)), f
     assert np.array_equal(ctx.trace_any(r), orc.trace_any(r))
+
+
+@pytest.mark.parametrize("ntri", [4, 1000, 30000])
+@pytest.mark.parametrize("tilt", [0.0, 1e-3])
+def test_rays_through_stacked_sheets_use_the_whole_stack(ntri, tilt):
+    """Parallel sheets that every ray crosses: all four children of a node are
+    hit on every level, so the stack grows by three entries a level, past the
+    entries kept in LDS.  Without tilt the rays are parallel to an axis (two
+    infinite components of 1/d)."""
+    print(f"[fetch] sheets {ntri} tilt {tilt}", flush=True)
+    rng = np.random.default_rng(ntri)
+    z = np.linspace(0.0, 1.0, ntri) + rng.uniform(0, 1e-6, ntri)
+    v = np.zeros((ntri, 3, 3))
+    v[:, 0, :2], v[:, 1, :2], v[:, 2, :2] = (-3, -3), (5, -3), (-3, 5)
+    v[:, :, 2] = z[:, None]
+    s = lfh.Scene()
+    s.add_material(lfh.MATERIAL_DEFAULT)
+    s.add_instance(s.add_mesh(v.astype(np.float32)), None, 0)
+    s.build()
+    n = 3000
+    r = np.zeros(n, lfh.RAY_DTYPE)
+    r["org"][:, :2] = rng.uniform(0.1, 0.4, (n, 2))
+    # half way between sheets: a ray starting in a sheet's plane enters its flat box only
+    # where the tree has grouped it with another (the distance is then 0)
+    r["org"][:, 2] = (rng.integers(-ntri // 5, ntri + ntri // 5, n) + 0.5) / (ntri - 1)
+    up = rng.random(n) < 0.5
+    d = np.stack([np.full(n, tilt), np.full(n, 2 * tilt), np.where(up, 1.0, -1.0)], 1)
+    r["dir"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    r["tmin"] = np.where(rng.random(n) < 0.3, 0.3, 0.0)     # hits behind tmin are passed over
+    r["tmax"] = scenes.RAY_TMAX
+    orc = native.OracleScene(s.arrays())
+    want, occ = orc.trace_closest(r), orc.trace_any(r)
+    for device_bvh in (False, True):
+        ctx = lfh.Context.from_scene(s, device_bvh=device_bvh)
+        got = ctx.trace_closest(r)
+        for f in ("prim", "inst"):
+            assert np.array_equal(got[f], want[f]), (f, device_bvh)
+        for f in ("t", "u", "v"):
+            assert np.array_equal(got[f].view(np.uint32), want[f].view(np.uint32)), (f, device_bvh)
+        assert np.array_equal(ctx.trace_any(r), occ), device_bvh
+        ctx.close()
