@@ -69,6 +69,22 @@ PathBufs view(const PassBufs& b) {
     return p;
 }
 
+PtQueues queues(const PassBufs& b, uint32_t* spill, int* err, int grid_blocks, float cull) {
+    PtQueues q;
+    q.rayq[0] = b.rq0.as<float4>();
+    q.rayq[1] = b.rq1.as<float4>();
+    q.hitq = b.hq.as<float4>();
+    q.shadowq = b.sq.as<float4>();
+    q.counts = b.counters.as<uint32_t>();
+    q.work = b.work.as<unsigned long long>();
+    q.spill = spill;
+    q.err = err;
+    q.maxq = b.cap;
+    q.grid_blocks = grid_blocks;
+    q.cull = cull;
+    return q;
+}
+
 }  // namespace lfh
 
 namespace lfh {
@@ -99,7 +115,6 @@ int render_init(lfh_ctx* c) {
         c->pt_grid = pt_trace_grid_blocks();
         size_t need = (size_t)c->pt_grid * lfh_trace_threads_per_block() * lfh_trace_spill_stride() * 4;
         if (need > c->spill.bytes) e = c->spill.alloc(need);
-        if (e == hipSuccess && shadow_lane_enabled()) e = c->lane.init(need);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return rhip(c, e, "render_init");
@@ -108,20 +123,11 @@ int render_init(lfh_ctx* c) {
 
 void render_release(lfh_ctx* c) {
     c->bgraph.reset();
-    c->lane.release();
 }
 
 bool bounce_graphs_enabled() {
     static const bool on = [] {
         const char* e = std::getenv("LFH_BOUNCE_GRAPHS");
-        return !(e && e[0] == '0');
-    }();
-    return on;
-}
-
-bool shadow_lane_enabled() {
-    static const bool on = [] {
-        const char* e = std::getenv("LFH_SHADOW_LANE");
         return !(e && e[0] == '0');
     }();
     return on;
@@ -194,25 +200,12 @@ int render_tile(lfh_ctx* c, int batch) {
     GuideHook gh{};
     lfhd::GuideDev gd{};
     if (guide_pass_begin(c, batch, &gh, &gd) < 0) return rfail(c, LFH_E_HIP, "render: guide buffers");
-    const ShadowLane lane = c->lane.lane();
-    const ShadowLane* lp = c->lane.ready() ? &lane : nullptr;
-    auto chain = [&]() -> hipError_t {
-        for (int depth = 0; depth < c->opt.max_depth; ++depth) {
-            const int cur = depth & 1;
-            float4* q[2] = {pb.rq0.as<float4>(), pb.rq1.as<float4>()};
-            hipError_t e = pt_bounce(sc, depth, pb.cap, q[cur], cnt + cur, q[cur ^ 1], cnt + (cur ^ 1),
-                                     pb.hq.as<float4>(), pb.sq.as<float4>(), cnt + 2, lfh::view(pb),
-                                     c->spill.as<uint32_t>(), work, c->rflag.as<int>(), c->cull, c->pt_grid, gh, &gd,
-                                     c->stream, lp);
-            if (e != hipSuccess) return e;
-        }
-        return lp && c->opt.max_depth > 0 ? pt_bounce_join(*lp, c->stream) : hipSuccess;
-    };
+    const PtQueues q = queues(pb, c->spill.as<uint32_t>(), c->rflag.as<int>(), c->pt_grid, c->cull);
+    auto chain = [&]() -> hipError_t { return pt_bounces(sc, c->opt.max_depth, q, lfh::view(pb), gh, &gd, c->stream); };
     if (!gh.enabled && bounce_graphs_enabled()) {
         // the guide hook changes every pass; unguided chains are replayed
         const std::vector<uintptr_t> key = {(uintptr_t)pb.rad.p,  (uintptr_t)pb.cap,     (uintptr_t)c->opt.max_depth,
-                                            (uintptr_t)c->stream, (uintptr_t)c->spill.p, (uintptr_t)c->scene_version,
-                                            (uintptr_t)c->lane.s, (uintptr_t)c->lane.spill.p};
+                                            (uintptr_t)c->stream, (uintptr_t)c->spill.p, (uintptr_t)c->scene_version};
         RCHK(c, run_graph(c->bgraph, key, c->stream, chain), "render: bounce graph");
     } else {
         RCHK(c, chain(), "render: bounce");
@@ -288,16 +281,9 @@ int render_preview(lfh_ctx* c, float scale, int dof, int* pw, int* ph) {
     unsigned long long* work = pb.work.as<unsigned long long>();
     RCHK(c, pt_reset(cnt, work, c->stream), "lfh_render_preview: reset");
     RCHK(c, pt_generate(cp, lfh::view(pb), pb.rq0.as<float4>(), cnt + 0, c->stream), "lfh_render_preview: generate");
-    GuideHook gh{};
-    for (int depth = 0; depth < o.max_depth; ++depth) {
-        const int cur = depth & 1;
-        float4* q[2] = {pb.rq0.as<float4>(), pb.rq1.as<float4>()};
-        RCHK(c,
-             pt_bounce(sc, depth, pb.cap, q[cur], cnt + cur, q[cur ^ 1], cnt + (cur ^ 1), pb.hq.as<float4>(),
-                       pb.sq.as<float4>(), cnt + 2, lfh::view(pb), c->spill.as<uint32_t>(), work, c->rflag.as<int>(),
-                       c->cull, c->pt_grid, gh, nullptr, c->stream),
-             "lfh_render_preview: bounce");
-    }
+    const PtQueues q = queues(pb, c->spill.as<uint32_t>(), c->rflag.as<int>(), c->pt_grid, c->cull);
+    RCHK(c, pt_bounces(sc, o.max_depth, q, lfh::view(pb), GuideHook{}, nullptr, c->stream),
+         "lfh_render_preview: bounce");
     lfhd::CamParams ca = cp;   // accumulate over the preview frame itself
     ca.width = W;
     ca.height = H;
@@ -398,6 +384,10 @@ int lfh_get_ray_counts(lfh_ctx* c, int64_t* extended, int64_t* shadow) {
     RCHK(c, hipMemcpyAsync(t, c->pass.work.as<unsigned long long>() + lfhd::kWorkTotals, sizeof t, hipMemcpyDeviceToHost, c->stream),
          "lfh_get_ray_counts");
     RCHK(c, hipStreamSynchronize(c->stream), "lfh_get_ray_counts");
+    // the rays of the last wavefront's last depths are not in the totals yet
+    uint32_t n[2 * lfhd::kQueueSets] = {};
+    RCHK(c, hipMemcpy(n, c->pass.counters.p, sizeof n, hipMemcpyDeviceToHost), "lfh_get_ray_counts");
+    for (int k = 0; k < 2 * lfhd::kQueueSets; ++k) t[k & 1] += n[k];
     *extended = (int64_t)t[0];
     *shadow = (int64_t)t[1];
     return LFH_OK;
@@ -630,16 +620,8 @@ int lfh_path_trace_rays(lfh_ctx* c, const float* rays6, uint32_t* seeds, int64_t
     RCHK(c, pt_reset(cnt, work, c->stream), fn);
     RCHK(c, pt_generate_rays(dr, ds, (int)n, lfh::view(pb), pb.rq0.as<float4>(), cnt, c->stream), fn);
     lfhd::ShadeScene sc = lfh::shade_view(c->ps, c->ds, c->opt);
-    GuideHook gh{};
-    for (int depth = 0; depth < c->opt.max_depth; ++depth) {
-        const int cur = depth & 1;
-        float4* q[2] = {pb.rq0.as<float4>(), pb.rq1.as<float4>()};
-        RCHK(c,
-             pt_bounce(sc, depth, pb.cap, q[cur], cnt + cur, q[cur ^ 1], cnt + (cur ^ 1), pb.hq.as<float4>(),
-                       pb.sq.as<float4>(), cnt + 2, lfh::view(pb), c->spill.as<uint32_t>(), work, c->rflag.as<int>(),
-                       c->cull, c->pt_grid, gh, nullptr, c->stream),
-             fn);
-    }
+    const PtQueues q = lfh::queues(pb, c->spill.as<uint32_t>(), c->rflag.as<int>(), c->pt_grid, c->cull);
+    RCHK(c, pt_bounces(sc, c->opt.max_depth, q, lfh::view(pb), GuideHook{}, nullptr, c->stream), fn);
     RCHK(c, pt_collect(lfh::view(pb), (int)n, dout, c->stream), fn);
     RCHK(c, hipMemcpyAsync(radiance, dout, n * 12, hipMemcpyDeviceToHost, c->stream), fn);
     RCHK(c, hipStreamSynchronize(c->stream), fn);

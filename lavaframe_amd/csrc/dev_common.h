@@ -68,16 +68,18 @@ LFH_HD uint32_t make_inst(uint32_t inst) { return kRefInstBit | inst; }
 #endif
 // Work counters of the persistent traversal kernels: a queue's ray ids are
 // split into kFetchSlices contiguous slices, each with its own counter
-// kFetchStride 64-bit words (256 B) from the next.  The path tracer's work
-// buffer holds the extend queue's counters, then the shadow queue's, then
-// two running ray totals at kWorkTotals.
+// kFetchStride 64-bit words (256 B) from the next.  A wavefront keeps
+// kQueueSets sets of queue counters in turn, depth d using set d % kQueueSets:
+// the ray counts (extension, shadow) and both queues' fetch counters; two
+// running ray totals follow the fetch counters at kWorkTotals.
 #ifndef LFH_FETCH_SLICES
 #define LFH_FETCH_SLICES 8
 #endif
 constexpr int kFetchSlices = LFH_FETCH_SLICES;
 constexpr int kFetchStride = 32;
 constexpr int kFetchWords = kFetchSlices * kFetchStride;
-constexpr int kWorkTotals = 2 * kFetchWords;
+constexpr int kQueueSets = 3;
+constexpr int kWorkTotals = kQueueSets * 2 * kFetchWords;
 constexpr int kWorkWords = kWorkTotals + 8;
 #ifndef LFH_TRACE_SLICE
 // 16 / 24 / 32 / 48 steps: 16.8M closest hits 5.90 / 5.92 / 5.92 / 6.09 ms, instanced 1080p frame

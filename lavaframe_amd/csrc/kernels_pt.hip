@@ -81,34 +81,23 @@ LFH_DEV uint32_t block_append(uint32_t* counter, bool want, uint32_t* lds) {
 
 LFH_DEV float4 f4(V3 v, float w) { return make_float4(v.x, v.y, v.z, w); }
 
-__global__ void k_pt_reset(uint32_t* counters, unsigned long long* work) {
-    int i = threadIdx.x;
-    if (i < 8) counters[i] = 0u;
-    if (i < 2 * kFetchSlices) work[i * kFetchStride] = 0ull;
+// Counter set of depth d: its counts and its queues' fetch counters.
+LFH_HD uint32_t* set_counts(uint32_t* counts, int d) { return counts + 2 * (d % kQueueSets); }
+LFH_HD unsigned long long* set_fetch(unsigned long long* work, int d) { return work + (size_t)(d % kQueueSets) * 2 * kFetchWords; }
+
+// Adds a set's ray counts to the running totals and clears the set (threads
+// 0 .. 2 kFetchSlices - 1 of one block).
+LFH_DEV void retire_set(uint32_t* counts, unsigned long long* fetch, unsigned long long* totals, int t) {
+    if (t < 2) {
+        totals[t] += counts[t];
+        counts[t] = 0u;
+    }
+    if (t < 2 * kFetchSlices) fetch[t * kFetchStride] = 0ull;
 }
 
-// work: the extend and shadow queues' fetch counters (zeroed after every
-// bounce), then at kWorkTotals the running totals of extended and shadow
-// rays (never reset by a pass).
-__global__ void k_pt_advance(uint32_t* consumed, uint32_t* shadow_count, unsigned long long* work) {
-    if (threadIdx.x == 0) {
-        work[kWorkTotals] += *consumed;
-        work[kWorkTotals + 1] += *shadow_count;
-        *consumed = 0u;
-        *shadow_count = 0u;
-    }
-    if (threadIdx.x < 2 * kFetchSlices) work[threadIdx.x * kFetchStride] = 0ull;
-}
-
-// One queue's half of k_pt_advance, for a chain whose shadow traversal runs
-// on its own stream: the queue's count goes to its running total, then the
-// count and the queue's fetch counters are cleared.
-__global__ void k_pt_advance_queue(uint32_t* count, unsigned long long* fetch, unsigned long long* total) {
-    if (threadIdx.x == 0) {
-        *total += *count;
-        *count = 0u;
-    }
-    if (threadIdx.x < kFetchSlices) fetch[threadIdx.x * kFetchStride] = 0ull;
+__global__ void k_pt_reset(uint32_t* counts, unsigned long long* work) {
+    for (int d = 0; d < kQueueSets; ++d)
+        retire_set(set_counts(counts, d), set_fetch(work, d), work + kWorkTotals, (int)threadIdx.x);
 }
 
 // generate: one thread per tile pixel (MULTI: per pixel of every job)
@@ -242,35 +231,22 @@ LFH_DEV bool light_any(const ShadeScene& sc, V3 o, V3 d, float maxDist) {
     return false;
 }
 
+// One wave's share of a ray queue: extension rays write hit records, shadow
+// rays clear the weight of their next-event term when they are occluded.
 template <bool SHADOW, bool MULTI>
-#ifndef LFH_QUEUE_WAVES
-#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD: 6 / 5: C0 3.10 / 3.26 ms, instanced 1080p frame 22.3 / 24.4 ms
-#endif
-__global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queue(ShadeScene sc, const JobDev* __restrict__ jobs,
-                                                             const float4* __restrict__ q,
-                                                             const uint32_t* __restrict__ count,
-                                                             float4* __restrict__ hitq, PathBufs pb,
-                                                             uint32_t* __restrict__ spill,
-                                                             unsigned long long* __restrict__ work, float cull,
-                                                             int* __restrict__ err) {
-    __shared__ uint32_t stk[kTraceBlock / 64][kLdsStack][64];
+LFH_DEV void trace_queue(const ShadeScene& sc, const JobDev* __restrict__ jobs, const float4* __restrict__ q,
+                         int64_t n, float4* __restrict__ hitq, const PathBufs& pb, LaneStack& st,
+                         unsigned long long* __restrict__ work, int block, float cull, int* __restrict__ err) {
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    LaneStack st;
-    st.lds = (LdsWord*)&stk[wave][0][lane];
-    st.spill = (GlobalWord*)(spill + gtid * kSpillStride);
-    st.reset();
-    const int64_t n = (int64_t)*count;
+    WaveFetch fetch;
+    fetch.init(n, (int)gridDim.x, kTraceBlock / 64, block, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    if (fetch.idle()) return;   // wave-uniform; the kernel has no block barrier
     TraceState s;
     bool active = false;
     int64_t rid = 0;
     int light = -1;
     float lpdf = 0.f;
     TraceScene ts = sc.tr;
-    WaveFetch fetch;
-    fetch.init(n, (int)gridDim.x, kTraceBlock / 64, (int)blockIdx.x, __builtin_amdgcn_readfirstlane(wave));
-    if (fetch.idle()) return;   // wave-uniform; the kernel has no block barrier
     for (;;) {
         const bool need = !active;
         const uint64_t mask = __ballot(need);
@@ -331,6 +307,36 @@ __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queue(Sh
             }
         }
     }
+}
+
+// Extension rays of one depth and shadow rays of the depth before, which do
+// not depend on each other, in one launch: a wave that finds no more extension
+// rays goes on with shadow rays, so the slowest extension rays and the shadow
+// traversal share the chip without a second stream.  The shadow queue's first
+// rays go to the waves in reverse order, so that in small wavefronts other
+// waves take them.
+#ifndef LFH_QUEUE_WAVES
+#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD: 6 / 5: C0 3.10 / 3.26 ms, instanced 1080p frame 22.3 / 24.4 ms
+#endif
+template <bool MULTI>
+__global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queues(ShadeScene sc, const JobDev* __restrict__ jobs,
+                                                              const float4* __restrict__ rayq, const uint32_t* __restrict__ rays,
+                                                              unsigned long long* __restrict__ ray_work,
+                                                              float4* __restrict__ hitq,
+                                                              const float4* __restrict__ shadowq,
+                                                              const uint32_t* __restrict__ shadows,
+                                                              unsigned long long* __restrict__ shadow_work, PathBufs pb,
+                                                              uint32_t* __restrict__ spill, float cull,
+                                                              int* __restrict__ err) {
+    __shared__ uint32_t stk[kTraceBlock / 64][kLdsStack][64];
+    LaneStack st;
+    st.lds = (LdsWord*)&stk[threadIdx.x >> 6][0][threadIdx.x & 63];
+    st.spill = (GlobalWord*)(spill + ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * kSpillStride);
+    st.reset();
+    const int block = (int)blockIdx.x;
+    trace_queue<false, MULTI>(sc, jobs, rayq, (int64_t)*rays, hitq, pb, st, ray_work, block, cull, err);
+    trace_queue<true, MULTI>(sc, jobs, shadowq, (int64_t)*shadows, hitq, pb, st, shadow_work,
+                             (int)gridDim.x - 1 - block, cull, err);
 }
 
 // ---- shade ------------------------------------------------------------------------
@@ -417,8 +423,12 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
                                                const float4* __restrict__ hitq, const uint32_t* __restrict__ count,
                                                float4* __restrict__ nextq, uint32_t* __restrict__ next_count,
                                                float4* __restrict__ shadowq, uint32_t* __restrict__ shadow_count,
-                                               PathBufs pb, GuideHook gh) {
+                                               PathBufs pb, GuideHook gh, uint32_t* __restrict__ done_counts,
+                                               unsigned long long* __restrict__ done_fetch,
+                                               unsigned long long* __restrict__ totals) {
     const uint32_t n = *count;
+    // the counters of the depth before are read by nothing any more
+    if (blockIdx.x == 0) retire_set(done_counts, done_fetch, totals, (int)threadIdx.x);
 #if LFH_SHADE_BIN
     __shared__ uint32_t bins[kShadeClasses * 4 + 256];
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -857,110 +867,49 @@ hipError_t pt_generate_rays(const float* rays6, const uint4* seeds, int n, const
     return hipGetLastError();
 }
 
-#ifndef LFH_LANE_GRID_NUM
-// the lane's shadow traversal launches this many quarters of the resident grid: 2 / 3 / 4 quarters
-// measured C0 1287.8 / 1255.5 / 1228.6 Msamples/s, C2 429.0 / 438.9 / 440.0, guided C3 pass
-// 2.217 / 2.113 / 2.072 ms
-#define LFH_LANE_GRID_NUM 4
-#endif
-#ifndef LFH_INFER_AFTER_SHADOW
-#define LFH_INFER_AFTER_SHADOW 0   // 1: guide inference waits for the shadow traversal too (median
-                                   // guided C3 time to 1e-2 over 32 sequences 0.158 s against 0.156)
-#endif
-// Shading of `depth` waits for the lane's shadow traversal of depth - 1.
-static hipError_t wait_shadowed(const ShadowLane* lane, int depth, hipStream_t s) {
-    return lane && depth > 0 ? hipStreamWaitEvent(s, lane->shadowed, 0) : hipSuccess;
-}
+namespace {
 
-// After shading: the extension queue's counters are reset on the main stream,
-// and the shadow traversal with its reset runs on the lane.
+// One wavefront's bounces: per depth one traversal launch (this depth's
+// extension rays, the last depth's shadow rays), guide inference for guided
+// wavefronts, and shading; a last traversal takes the last shadow rays.
 template <bool MULTI>
-static hipError_t shadow_on_lane(const ShadeScene& sc, const JobDev* jobs, uint32_t* count, float4* hitq,
-                                 float4* shadowq, uint32_t* shadow_count, const PathBufs& pb,
-                                 unsigned long long* work, int* err, float cull, int grid_blocks,
-                                 const ShadowLane& lane, hipStream_t s) {
-    hipLaunchKernelGGL(k_pt_advance_queue, dim3(1), dim3(64), 0, s, count, work, work + kWorkTotals);
-    hipError_t e = hipEventRecord(lane.shaded, s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(lane.s, lane.shaded, 0);
-    if (e != hipSuccess) return e;
-    const int lane_blocks = grid_blocks * LFH_LANE_GRID_NUM / 4 > 0 ? grid_blocks * LFH_LANE_GRID_NUM / 4 : 1;
-    hipLaunchKernelGGL((k_trace_queue<true, MULTI>), dim3(lane_blocks), dim3(kTraceBlock), 0, lane.s, sc, jobs,
-                       shadowq, shadow_count, hitq, pb, lane.spill, work + kFetchWords, cull, err);
-    hipLaunchKernelGGL(k_pt_advance_queue, dim3(1), dim3(64), 0, lane.s, shadow_count, work + kFetchWords,
-                       work + kWorkTotals + 1);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipEventRecord(lane.shadowed, lane.s);
-    return e;
-}
-
-hipError_t pt_bounce_join(const ShadowLane& lane, hipStream_t s) { return hipStreamWaitEvent(s, lane.shadowed, 0); }
-
-hipError_t pt_bounce(const ShadeScene& sc, int depth, int maxq, float4* rayq, uint32_t* count, float4* nextq,
-                     uint32_t* next_count, float4* hitq, float4* shadowq, uint32_t* shadow_count, const PathBufs& pb,
-                     uint32_t* spill, unsigned long long* work, int* err, float cull, int grid_blocks,
-                     const GuideHook& gh, const lfhd::GuideDev* gd, hipStream_t s, const ShadowLane* lane) {
-    const JobDev* nj = nullptr;
-    hipLaunchKernelGGL((k_trace_queue<false, false>), dim3(grid_blocks), dim3(kTraceBlock), 0, s, sc, nj, rayq, count,
-                       hitq, pb, spill, work, cull, err);
-    if (LFH_INFER_AFTER_SHADOW && gh.enabled) {
-        hipError_t e = wait_shadowed(lane, depth, s);
-        if (e != hipSuccess) return e;
+hipError_t bounces(const ShadeScene& sc, const JobDev* jobs, int max_depth, const PtQueues& q, const PathBufs& pb,
+                   const GuideHook& gh, const lfhd::GuideDev* gd, const ShadeScene& guide_sc, hipStream_t s) {
+    if (max_depth <= 0) return hipSuccess;
+    for (int d = 0;; ++d) {
+        const int last = d + kQueueSets - 1;   // same set as depth d - 1
+        uint32_t* rays = set_counts(q.counts, d);
+        hipLaunchKernelGGL((k_trace_queues<MULTI>), dim3(q.grid_blocks), dim3(kTraceBlock), 0, s, sc, jobs,
+                           q.rayq[d & 1], rays, set_fetch(q.work, d), q.hitq, q.shadowq,
+                           set_counts(q.counts, last) + 1, set_fetch(q.work, last) + kFetchWords, pb, q.spill, q.cull,
+                           q.err);
+        if (d == max_depth) break;
+        if (gh.enabled) {
+            hipError_t e = guide_infer_queue(*gd, guide_sc, q.rayq[d & 1], q.hitq, rays, q.maxq, gh, d,
+                                             const_cast<float4*>(gh.lobes), s);
+            if (e != hipSuccess) return e;
+        }
+        const auto shade = gh.enabled ? k_shade<MULTI, true> : k_shade<MULTI, false>;
+        hipLaunchKernelGGL(shade, dim3(nblk(q.maxq)), dim3(256), 0, s, sc, jobs, d, q.rayq[d & 1], q.hitq, rays,
+                           q.rayq[(d + 1) & 1], set_counts(q.counts, d + 1), q.shadowq, rays + 1, pb, gh,
+                           set_counts(q.counts, last), set_fetch(q.work, last), q.work + kWorkTotals);
     }
-    if (gh.enabled) {
-        hipError_t e = guide_infer_queue(*gd, sc, rayq, hitq, count, maxq, gh, depth,
-                                         const_cast<float4*>(gh.lobes), s);
-        if (e != hipSuccess) return e;
-    }
-    hipError_t e = wait_shadowed(lane, depth, s);
-    if (e != hipSuccess) return e;
-    if (gh.enabled)
-        hipLaunchKernelGGL((k_shade<false, true>), dim3(nblk(maxq)), dim3(256), 0, s, sc, nj, depth, rayq, hitq, count,
-                           nextq, next_count, shadowq, shadow_count, pb, gh);
-    else
-        hipLaunchKernelGGL((k_shade<false, false>), dim3(nblk(maxq)), dim3(256), 0, s, sc, nj, depth, rayq, hitq, count,
-                           nextq, next_count, shadowq, shadow_count, pb, gh);
-    if (lane)
-        return shadow_on_lane<false>(sc, nj, count, hitq, shadowq, shadow_count, pb, work, err, cull, grid_blocks,
-                                     *lane, s);
-    hipLaunchKernelGGL((k_trace_queue<true, false>), dim3(grid_blocks), dim3(kTraceBlock), 0, s, sc, nj, shadowq,
-                       shadow_count, hitq, pb, spill, work + kFetchWords, cull, err);
-    hipLaunchKernelGGL(k_pt_advance, dim3(1), dim3(64), 0, s, count, shadow_count, work);
     return hipGetLastError();
 }
 
-hipError_t pt_bounce_multi(const JobDev* jobs, int depth, int maxq, float4* rayq, uint32_t* count, float4* nextq,
-                           uint32_t* next_count, float4* hitq, float4* shadowq, uint32_t* shadow_count,
-                           const PathBufs& pb, uint32_t* spill, unsigned long long* work, int* err, float cull,
-                           int grid_blocks, const GuideHook& gh, const lfhd::GuideDev* gd, const ShadeScene* guide_sc,
-                           hipStream_t s, const ShadowLane* lane) {
-    ShadeScene dummy{};
-    hipLaunchKernelGGL((k_trace_queue<false, true>), dim3(grid_blocks), dim3(kTraceBlock), 0, s, dummy, jobs, rayq,
-                       count, hitq, pb, spill, work, cull, err);
-    if (LFH_INFER_AFTER_SHADOW && gh.enabled) {
-        hipError_t e = wait_shadowed(lane, depth, s);
-        if (e != hipSuccess) return e;
-    }
-    if (gh.enabled) {
-        // every job of a guided wavefront draws on one scene (the guide's)
-        hipError_t e = guide_infer_queue(*gd, *guide_sc, rayq, hitq, count, maxq, gh, depth,
-                                         const_cast<float4*>(gh.lobes), s);
-        if (e != hipSuccess) return e;
-    }
-    hipError_t e = wait_shadowed(lane, depth, s);
-    if (e != hipSuccess) return e;
-    if (gh.enabled)
-        hipLaunchKernelGGL((k_shade<true, true>), dim3(nblk(maxq)), dim3(256), 0, s, dummy, jobs, depth, rayq, hitq,
-                           count, nextq, next_count, shadowq, shadow_count, pb, gh);
-    else
-        hipLaunchKernelGGL((k_shade<true, false>), dim3(nblk(maxq)), dim3(256), 0, s, dummy, jobs, depth, rayq, hitq,
-                           count, nextq, next_count, shadowq, shadow_count, pb, gh);
-    if (lane)
-        return shadow_on_lane<true>(dummy, jobs, count, hitq, shadowq, shadow_count, pb, work, err, cull,
-                                    grid_blocks, *lane, s);
-    hipLaunchKernelGGL((k_trace_queue<true, true>), dim3(grid_blocks), dim3(kTraceBlock), 0, s, dummy, jobs, shadowq,
-                       shadow_count, hitq, pb, spill, work + kFetchWords, cull, err);
-    hipLaunchKernelGGL(k_pt_advance, dim3(1), dim3(64), 0, s, count, shadow_count, work);
-    return hipGetLastError();
+}  // namespace
+
+hipError_t pt_bounces(const ShadeScene& sc, int max_depth, const PtQueues& q, const PathBufs& pb, const GuideHook& gh,
+                      const lfhd::GuideDev* gd, hipStream_t s) {
+    return bounces<false>(sc, nullptr, max_depth, q, pb, gh, gd, sc, s);
+}
+
+hipError_t pt_bounces_multi(const JobDev* jobs, int max_depth, const PtQueues& q, const PathBufs& pb,
+                            const GuideHook& gh, const lfhd::GuideDev* gd, const ShadeScene* guide_sc,
+                            hipStream_t s) {
+    // every job of a guided wavefront draws on one scene (the guide's)
+    const ShadeScene none{};
+    return bounces<true>(none, jobs, max_depth, q, pb, gh, gd, guide_sc ? *guide_sc : none, s);
 }
 
 hipError_t pt_accumulate_multi(const JobDev* jobs, int total, const PathBufs& pb, hipStream_t s) {
@@ -1006,10 +955,10 @@ int pt_trace_grid_blocks() {
         hipGetDevice(&dev);
         hipDeviceProp_t prop;
         hipGetDeviceProperties(&prop, dev);
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, (const void*)k_trace_queue<false, true>, kTraceBlock, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, (const void*)k_trace_queues<true>, kTraceBlock, 0) !=
                 hipSuccess || a <= 0)
             a = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, (const void*)k_trace_queue<false, false>, kTraceBlock, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, (const void*)k_trace_queues<false>, kTraceBlock, 0) !=
                 hipSuccess || b <= 0)
             b = 4;
         blocks = (a > b ? a : b) * prop.multiProcessorCount;

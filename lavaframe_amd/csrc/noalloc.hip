@@ -101,26 +101,26 @@ extern "C" int lfh_path_trace_rays_device_noalloc(lfh_ctx* c, const float* d_ray
     pb.rng = reinterpret_cast<uint4*>(take(kF4));
     pb.misc = reinterpret_cast<float4*>(take(kF4));
     pb.nee = reinterpret_cast<float4*>(take(3 * kF4));
-    float4* rq0 = reinterpret_cast<float4*>(take(2 * kF4));
-    float4* rq1 = reinterpret_cast<float4*>(take(2 * kF4));
-    float4* hq = reinterpret_cast<float4*>(take(2 * kF4));
-    float4* sq = reinterpret_cast<float4*>(take(4 * kF4));
+    PtQueues q;
+    q.rayq[0] = reinterpret_cast<float4*>(take(2 * kF4));
+    q.rayq[1] = reinterpret_cast<float4*>(take(2 * kF4));
+    q.hitq = reinterpret_cast<float4*>(take(2 * kF4));
+    q.shadowq = reinterpret_cast<float4*>(take(4 * kF4));
     pb.job = reinterpret_cast<int*>(take((size_t)kNoAllocPaths * 4));
-    uint32_t* cnt = reinterpret_cast<uint32_t*>(take(kCountersBytes));
-    unsigned long long* work = reinterpret_cast<unsigned long long*>(take(kWorkBytes));
+    q.counts = reinterpret_cast<uint32_t*>(take(kCountersBytes));
+    q.work = reinterpret_cast<unsigned long long*>(take(kWorkBytes));
+    q.spill = c->spill.as<uint32_t>();
+    q.err = c->rflag.as<int>();
+    q.maxq = (int)kNoAllocPaths;
+    q.grid_blocks = c->pt_grid;
+    q.cull = c->cull;
     if (off > kScratchBytes) return fail(c, LFH_E_INVALID, std::string(fn) + ": scratch layout exceeds its size");
-    const int cap = (int)kNoAllocPaths;
-    hipError_t e = pt_reset(cnt, work, c->stream);   // counters start at zero (a kernel, no memset)
+    hipError_t e = pt_reset(q.counts, q.work, c->stream);   // counters start at zero (a kernel, no memset)
     if (e == hipSuccess)
-        e = pt_generate_rays(d_rays6, reinterpret_cast<const uint4*>(d_seeds), (int)n, pb, rq0, cnt, c->stream);
-    lfhd::ShadeScene sc = lfh::shade_view(c->ps, c->ds, c->opt);
-    GuideHook gh{};
-    for (int depth = 0; e == hipSuccess && depth < c->opt.max_depth; ++depth) {
-        const int cur = depth & 1;
-        float4* q[2] = {rq0, rq1};
-        e = pt_bounce(sc, depth, cap, q[cur], cnt + cur, q[cur ^ 1], cnt + (cur ^ 1), hq, sq, cnt + 2, pb,
-                      c->spill.as<uint32_t>(), work, c->rflag.as<int>(), c->cull, c->pt_grid, gh, nullptr, c->stream);
-    }
+        e = pt_generate_rays(d_rays6, reinterpret_cast<const uint4*>(d_seeds), (int)n, pb, q.rayq[0], q.counts,
+                             c->stream);
+    const lfhd::ShadeScene sc = lfh::shade_view(c->ps, c->ds, c->opt);
+    if (e == hipSuccess) e = pt_bounces(sc, c->opt.max_depth, q, pb, GuideHook{}, nullptr, c->stream);
     if (e == hipSuccess) e = pt_collect(pb, (int)n, d_radiance, c->stream);
     if (e != hipSuccess)
         return fail(c, e == hipErrorOutOfMemory ? LFH_E_OOM : LFH_E_HIP, std::string(fn) + ": " + hipGetErrorString(e));

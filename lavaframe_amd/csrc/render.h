@@ -15,6 +15,8 @@ hipError_t run_graph(BounceGraph& g, const std::vector<uintptr_t>& key, hipStrea
 void render_release(lfh_ctx* c);
 // Device views of a pass's path buffers.
 PathBufs view(const PassBufs& b);
+// A pass's queues, traversed by grid_blocks blocks with these stacks.
+PtQueues queues(const PassBufs& b, uint32_t* spill, int* err, int grid_blocks, float cull);
 // Learned-guide hooks of one pass: begin fills the hook and the weights view
 // (returns 1 when a guide is attached, 0 if not, -1 on a HIP error); end
 // collects the pass's training samples and runs the optimisation steps.
