@@ -63,9 +63,10 @@ PathBufs view(const PassBufs& b) {
     p.thr = b.thr.as<float4>();
     p.absorb = b.absorb.as<float4>();
     p.rng = b.rng.as<uint4>();
-    p.misc = b.misc.as<float4>();
+    p.texc = b.texc.as<float2>();
     p.nee = b.nee.as<float4>();
     p.job = b.job.as<int>();
+    p.stride = b.cap;
     return p;
 }
 
@@ -196,7 +197,7 @@ int render_tile(lfh_ctx* c, int batch) {
     uint32_t* cnt = pb.counters.as<uint32_t>();
     unsigned long long* work = pb.work.as<unsigned long long>();
     RCHK(c, pt_reset(cnt, work, c->stream), "render: reset");
-    RCHK(c, pt_generate(cp, lfh::view(pb), pb.rq0.as<float4>(), cnt + 0, c->stream), "render: generate");
+    RCHK(c, pt_generate(cp, c->opt.max_depth, lfh::view(pb), pb.rq0.as<float4>(), cnt + 0, c->stream), "render: generate");
     GuideHook gh{};
     lfhd::GuideDev gd{};
     if (guide_pass_begin(c, batch, &gh, &gd) < 0) return rfail(c, LFH_E_HIP, "render: guide buffers");
@@ -210,7 +211,8 @@ int render_tile(lfh_ctx* c, int batch) {
     } else {
         RCHK(c, chain(), "render: bounce");
     }
-    RCHK(c, pt_accumulate(lfh::view(pb), cp, c->rs.accum.as<float4>(), c->rs.comp.as<float4>(), c->opt.kahan, c->stream),
+    RCHK(c, pt_accumulate(lfh::view(pb), cp, c->rs.accum.as<float4>(), c->rs.comp.as<float4>(), c->opt.kahan, gh.train != 0,
+                          c->stream),
          "render: accumulate");
     int gr = guide_pass_end(c, gh, batch);
     if (gr != LFH_OK) return rfail(c, gr, std::string("render: ") + lfh_internal::thread_error());
@@ -280,14 +282,15 @@ int render_preview(lfh_ctx* c, float scale, int dof, int* pw, int* ph) {
     uint32_t* cnt = pb.counters.as<uint32_t>();
     unsigned long long* work = pb.work.as<unsigned long long>();
     RCHK(c, pt_reset(cnt, work, c->stream), "lfh_render_preview: reset");
-    RCHK(c, pt_generate(cp, lfh::view(pb), pb.rq0.as<float4>(), cnt + 0, c->stream), "lfh_render_preview: generate");
+    RCHK(c, pt_generate(cp, o.max_depth, lfh::view(pb), pb.rq0.as<float4>(), cnt + 0, c->stream),
+         "lfh_render_preview: generate");
     const PtQueues q = queues(pb, c->spill.as<uint32_t>(), c->rflag.as<int>(), c->pt_grid, c->cull);
     RCHK(c, pt_bounces(sc, o.max_depth, q, lfh::view(pb), GuideHook{}, nullptr, c->stream),
          "lfh_render_preview: bounce");
     lfhd::CamParams ca = cp;   // accumulate over the preview frame itself
     ca.width = W;
     ca.height = H;
-    RCHK(c, pt_accumulate(lfh::view(pb), ca, c->preview.as<float4>(), c->preview.as<float4>(), 0, c->stream),
+    RCHK(c, pt_accumulate(lfh::view(pb), ca, c->preview.as<float4>(), c->preview.as<float4>(), 0, false, c->stream),
          "lfh_render_preview: output");
     *pw = W;
     *ph = H;
@@ -618,7 +621,7 @@ int lfh_path_trace_rays(lfh_ctx* c, const float* rays6, uint32_t* seeds, int64_t
     uint32_t* cnt = pb.counters.as<uint32_t>();
     unsigned long long* work = pb.work.as<unsigned long long>();
     RCHK(c, pt_reset(cnt, work, c->stream), fn);
-    RCHK(c, pt_generate_rays(dr, ds, (int)n, lfh::view(pb), pb.rq0.as<float4>(), cnt, c->stream), fn);
+    RCHK(c, pt_generate_rays(dr, ds, (int)n, c->opt.max_depth, lfh::view(pb), pb.rq0.as<float4>(), cnt, c->stream), fn);
     lfhd::ShadeScene sc = lfh::shade_view(c->ps, c->ds, c->opt);
     const PtQueues q = lfh::queues(pb, c->spill.as<uint32_t>(), c->rflag.as<int>(), c->pt_grid, c->cull);
     RCHK(c, pt_bounces(sc, c->opt.max_depth, q, lfh::view(pb), GuideHook{}, nullptr, c->stream), fn);

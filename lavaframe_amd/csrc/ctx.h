@@ -139,7 +139,7 @@ struct RenderState {
 
 // Path state + queues of one wavefront pass for up to `cap` paths.
 struct PassBufs {
-    DevBuf rad, thr, absorb, rng, misc, nee;  // per path (nee: 3 float4)
+    DevBuf rad, thr, absorb, rng, texc, nee;  // per path (nee: 3 float4)
     DevBuf rq0, rq1, hq, sq;                  // ray queues, hit queue, shadow queue
     DevBuf counters, work;
     DevBuf job;                               // int per path (multi-job passes)
@@ -158,12 +158,12 @@ struct PassBufs {
         return hipSuccess;
     }
     void release() {
-        DevBuf* b[13] = {&rad, &thr, &absorb, &rng, &misc, &nee, &rq0, &rq1, &hq, &sq, &counters, &work, &job};
+        DevBuf* b[13] = {&rad, &thr, &absorb, &rng, &texc, &nee, &rq0, &rq1, &hq, &sq, &counters, &work, &job};
         for (DevBuf* x : b) x->release();
         cap = 0;
     }
     size_t bytes() const {
-        return rad.bytes + thr.bytes + absorb.bytes + rng.bytes + misc.bytes + nee.bytes + rq0.bytes + rq1.bytes +
+        return rad.bytes + thr.bytes + absorb.bytes + rng.bytes + texc.bytes + nee.bytes + rq0.bytes + rq1.bytes +
                hq.bytes + sq.bytes + counters.bytes + work.bytes + job.bytes;
     }
 
@@ -172,7 +172,7 @@ private:
         if (lfh_internal::inject_fault(lfh_internal::kFaultPathAlloc)) return hipErrorOutOfMemory;
         hipError_t e;
         const size_t f4 = 16;
-        DevBuf* b[10] = {&rad, &thr, &absorb, &rng, &misc, &nee, &rq0, &rq1, &hq, &sq};
+        DevBuf* b[10] = {&rad, &thr, &absorb, &rng, &texc, &nee, &rq0, &rq1, &hq, &sq};
         const size_t m[10] = {1, 1, 1, 1, 1, 3, 2, 2, 2, 4};
         for (int i = 0; i < 10; ++i)
             if ((e = b[i]->alloc(f4 * m[i] * (size_t)n)) != hipSuccess) return e;

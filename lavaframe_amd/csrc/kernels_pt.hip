@@ -29,21 +29,6 @@ LFH_DEV float* guide_rec(const GuideHook& g, int p, int depth) {
 }
 
 // ---- queue helpers ---------------------------------------------------------------
-#ifndef LFH_BLOCK_APPEND
-#define LFH_BLOCK_APPEND 1   // 1: queue appends take one atomic per block, 0: one per wave
-#endif
-// Wave-aggregated append: returns this lane's slot (valid only if `want`).
-LFH_DEV uint32_t wave_append(uint32_t* counter, bool want) {
-    const uint64_t mask = __ballot(want);
-    if (mask == 0) return 0;
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    return base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-}
-
 // Block-aggregated appends: every thread of the block calls them at the same
 // point (the kernels using them have no early exit).  One atomic per block
 // instead of one per wave: all the device's appends to a queue hit the same
@@ -100,11 +85,12 @@ __global__ void k_pt_reset(uint32_t* counts, unsigned long long* work) {
         retire_set(set_counts(counts, d), set_fetch(work, d), work + kWorkTotals, (int)threadIdx.x);
 }
 
-// generate: one thread per tile pixel (MULTI: per pixel of every job)
+// generate: one thread per tile pixel (MULTI: per pixel of every job).
+// unshaded: no depth will be shaded (path depth 0), so the radiance starts here.
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_generate(CamParams cam1, const JobDev* __restrict__ jobs, int njobs,
                                                   int total, PathBufs pb, float4* __restrict__ rayq,
-                                                  uint32_t* __restrict__ count) {
+                                                  uint32_t* __restrict__ count, int unshaded) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     int lp = p, j = 0;
     CamParams cam = cam1;
@@ -136,22 +122,12 @@ __global__ __launch_bounds__(256) void k_generate(CamParams cam1, const JobDev* 
             camera_ray_preview(cam, lx, ly, o, d, seed);
         else
             camera_ray(cam, lx, ly, o, d, seed);
-        pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-        pb.thr[p] = make_float4(1.f, 1.f, 1.f, 0.f);
-        pb.absorb[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+        // shading of depth 0 starts the rest of the path state
         pb.rng[p] = seed;
-        pb.misc[p] = make_float4(0.f, __int_as_float(0), 0.f, 0.f);
-        pb.nee[p * 3 + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
-    } else if (inrange) {
-        pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-        pb.nee[p * 3 + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (unshaded) pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-#if LFH_BLOCK_APPEND
     __shared__ uint32_t app[16];
     uint32_t slot = block_append(count, valid, app);
-#else
-    uint32_t slot = wave_append(count, valid);
-#endif
     if (valid) {
         rayq[(size_t)slot * 2] = f4(o, __int_as_float(p));
         rayq[(size_t)slot * 2 + 1] = f4(d, 0.f);
@@ -161,23 +137,15 @@ __global__ __launch_bounds__(256) void k_generate(CamParams cam1, const JobDev* 
 // generate from caller-given rays and seeds (lfh_path_trace_rays)
 __global__ __launch_bounds__(256) void k_generate_rays(const float* __restrict__ rays6, const uint4* __restrict__ seeds,
                                                        int n, PathBufs pb, float4* __restrict__ rayq,
-                                                       uint32_t* __restrict__ count) {
+                                                       uint32_t* __restrict__ count, int unshaded) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     bool valid = p < n;
     if (valid) {
-        pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-        pb.thr[p] = make_float4(1.f, 1.f, 1.f, 0.f);
-        pb.absorb[p] = make_float4(0.f, 0.f, 0.f, 0.f);
         pb.rng[p] = seeds[p];
-        pb.misc[p] = make_float4(0.f, __int_as_float(0), 0.f, 0.f);
-        pb.nee[p * 3 + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (unshaded) pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-#if LFH_BLOCK_APPEND
     __shared__ uint32_t app[16];
     uint32_t slot = block_append(count, valid, app);
-#else
-    uint32_t slot = wave_append(count, valid);
-#endif
     if (valid) {
         const float* r = rays6 + (size_t)p * 6;
         rayq[(size_t)slot * 2] = make_float4(r[0], r[1], r[2], __int_as_float(p));
@@ -289,7 +257,7 @@ LFH_DEV void trace_queue(const ShadeScene& sc, const JobDev* __restrict__ jobs, 
                         float4 a = q[rid * 2];
                         uint32_t tag = __float_as_uint(a.w);
                         uint32_t p = tag >> 1, kind = tag & 1u;
-                        pb.nee[(size_t)p * 3 + kind].w = 0.0f;
+                        pb.nee[(size_t)kind * pb.stride + p].w = 0.0f;
                     }
                 } else {
                     float4 h0, h1;
@@ -340,84 +308,46 @@ __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queues(S
 }
 
 // ---- shade ------------------------------------------------------------------------
-LFH_DEV void combine_nee(PathBufs& pb, int p, V3& rad) {
-    float4 tn = pb.nee[(size_t)p * 3 + 2];
-    if (tn.w != 0.0f) {
-        float4 e = pb.nee[(size_t)p * 3 + 0], l = pb.nee[(size_t)p * 3 + 1];
+// State word of a path (rad.w): the last surface's material, whether a
+// Beer-Lambert coefficient is stored, and which next-event terms of the last
+// vertex wait for their shadow rays.
+constexpr uint32_t kStateMat = 0x1FFFFFFFu, kStateLight = 1u << 29, kStateEnv = 1u << 30, kStateAbsorb = 1u << 31;
+
+// Adds the last vertex's next-event terms (weight 0 once their shadow ray met
+// something).  A vertex with one term stores it times the throughput; one
+// with both stores them as they are, and the throughput.
+LFH_DEV void combine_nee(const PathBufs& pb, int p, uint32_t word, V3& rad) {
+    const float4* env = pb.nee + p;
+    const float4* light = env + pb.stride;
+    if ((word & kStateEnv) && (word & kStateLight)) {
+        const float4 e = *env, l = *light, tn = light[pb.stride];
         V3 Li = v3(0.f, 0.f, 0.f);
         if (e.w != 0.0f) Li = Li + ld3(e);
         if (l.w != 0.0f) Li = Li + ld3(l);
         rad = rad + Li * ld3(tn);
-        pb.nee[(size_t)p * 3 + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
+    } else if (word & (kStateEnv | kStateLight)) {
+        const float4 c = word & kStateEnv ? *env : *light;
+        if (c.w != 0.0f) rad = rad + ld3(c);
     }
-}
-
-// Shading class of hit-queue entry i (miss, light, then the material's
-// dominant lobe group), for binning a block's entries before shading.
-#ifndef LFH_SHADE_BIN
-#define LFH_SHADE_BIN 0   // 1: a block shades its entries grouped by class (C2: 388.1 binned vs 390.6 Msamples/s; C0 unchanged)
-#endif
-constexpr int kShadeClasses = 6;
-template <bool MULTI>
-LFH_DEV int shade_class(const ShadeScene& sc1, const JobDev* jobs, const PathBufs& pb, const float4* rayq,
-                        const float4* hitq, uint32_t i, uint32_t n) {
-    if (i >= n) return kShadeClasses - 1;
-    const float4 h0 = hitq[(size_t)i * 2], h1 = hitq[(size_t)i * 2 + 1];
-    if (h0.x == kInfinity) return 0;
-    if (__float_as_int(h0.w) < 0) return 1;
-    const int p = __float_as_int(rayq[(size_t)i * 2].w);
-    const ShadeScene& sc = MULTI ? jobs[pb.job[p]].sc : sc1;
-    const float4* m = sc.materials + (size_t)__float_as_int(h1.y) * kMaterialF4;
-    const float metallic = m[2].x, trans = m[4].x;
-    if (trans > 0.0f && metallic < 1.0f) return 2;
-    return metallic >= 1.0f ? 3 : 4;
-}
-
-// Block-local counting sort of the entries by class: returns the entry this
-// thread shades.  Every entry of the block is shaded exactly once; a path's
-// result does not depend on which thread shades it (each entry updates only
-// its own path), so the permutation changes only the order of the appended
-// rays.  `lds` holds kShadeClasses * 4 + 256 words.
-LFH_DEV uint32_t bin_by_class(int cls, uint32_t* lds) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t rank = 0;
-#pragma unroll
-    for (int c = 0; c < kShadeClasses; ++c) {
-        const uint64_t m = __ballot(cls == c);
-        if (lane == 0) lds[c * 4 + wave] = (uint32_t)__popcll(m);
-        if (cls == c) rank = (uint32_t)__popcll(m & below);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int c = 0; c < kShadeClasses; ++c)
-            for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-                const uint32_t k = lds[c * 4 + w];
-                lds[c * 4 + w] = run;
-                run += k;
-            }
-    }
-    __syncthreads();
-    uint32_t* perm = lds + kShadeClasses * 4;
-    perm[lds[cls * 4 + wave] + rank] = threadIdx.x;
-    __syncthreads();
-    const uint32_t j = perm[threadIdx.x];
-    __syncthreads();
-    return j;
 }
 
 // GUIDED: the variant for guided wavefronts (guide sampling, MIS with the
 // guide's pdf, training records); unguided wavefronts run the variant without
 // that code, which would otherwise hold registers they never use.
-template <bool MULTI, bool GUIDED>
+//
+// Bound by the path state's and the queues' traffic on full queues and by one
+// chain of dependent loads and arithmetic on small ones.  Per path and bounce
+// of a scene with lights only and no media it moves 144 B in and up to 144 B
+// out (192 and 208 B with every array read and written, and 128 B per path
+// more by generation): C0 3.07 -> 2.88 ms, guiding room 8.20 -> 7.53 ms,
+// instanced 1080p 22.0 -> 20.7 ms, guided frame 14.0 -> 12.7 ms.  Budgeted for
+// 3 waves per SIMD (142-167 VGPRs).  Blocks that loop over the queue
+// (1536-8192 of them, sparing late depths their empty blocks) need 168 VGPRs with
+// spills: C0 2.91-2.95 ms, instanced 21.0-21.2 ms.
 #ifndef LFH_SHADE_WAVES
-// k_shade register budget in waves per SIMD.  1 (153-158 VGPRs, 3 waves): C0 1207 /
-// C2 391 Msamples/s, C3 1.463 / 2.134 ms per plain / guided pass; 4 (128 VGPRs,
-// 100-140 B/lane spilled): 1208 / 384, 1.506 / 2.216; 5 (96 VGPRs, 244-276 B):
-// 1037 / 363, 1.607 / 2.358.  The spills cost more than the occupancy gains.
-#define LFH_SHADE_WAVES 1
+#define LFH_SHADE_WAVES 3
 #endif
+template <bool MULTI, bool GUIDED>
 __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, const JobDev* __restrict__ jobs, int depth,
                                                const float4* __restrict__ rayq,
                                                const float4* __restrict__ hitq, const uint32_t* __restrict__ count,
@@ -429,15 +359,10 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
     const uint32_t n = *count;
     // the counters of the depth before are read by nothing any more
     if (blockIdx.x == 0) retire_set(done_counts, done_fetch, totals, (int)threadIdx.x);
-#if LFH_SHADE_BIN
-    __shared__ uint32_t bins[kShadeClasses * 4 + 256];
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if ((uint32_t)blockIdx.x * blockDim.x < n)   // block-uniform: blocks past the queue keep their order
-        i = blockIdx.x * blockDim.x +
-            bin_by_class(shade_class<MULTI>(sc1, jobs, pb, rayq, hitq, i, n), bins);
-#else
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-#endif
+    __shared__ uint32_t app[16];
+    const uint32_t base = blockIdx.x * 256u;
+    if (base >= n) return;   // block-uniform
+    const uint32_t i = base + threadIdx.x;
     const bool live = i < n;
     bool cont = false;
     bool shEnv = false, shLight = false;
@@ -451,15 +376,24 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
         const ShadeScene& sc = MULTI ? jobs[pb.job[p]].sc : sc1;
         V3 ro = ld3(r0), rd = ld3(r1);
         float4 h0 = hitq[(size_t)i * 2], h1 = hitq[(size_t)i * 2 + 1];
-        V3 rad = ld3(pb.rad[p]);
-        V3 thr = ld3(pb.thr[p]);
-        combine_nee(pb, p, rad);
+        // a path starts with no radiance and throughput 1
+        V3 rad = v3(0.f, 0.f, 0.f), thr = v3(1.f, 1.f, 1.f);
+        float prevPdf = 0.f;
+        uint32_t word = 0u;
+        float2 texc = make_float2(0.f, 0.f);   // last surface's texture coordinate
+        if (depth > 0) {
+            const float4 r4 = pb.rad[p], t4 = pb.thr[p];
+            rad = ld3(r4);
+            thr = ld3(t4);
+            prevPdf = t4.w;
+            word = __float_as_uint(r4.w);
+            if (sc.tex) texc = pb.texc[p];
+            combine_nee(pb, p, word, rad);
+        }
         const bool recorded = GUIDED && gh.train && (p % gh.stride) == gh.phase;
         if (recorded && depth > 0) guide_rec(gh, p, depth - 1)[11] = luminance(rad);
-        float4 misc = pb.misc[p];
-        float prevPdf = misc.x;
-        int lastMat = __float_as_int(misc.y);
-        float2 texc = make_float2(misc.z, misc.w);   // last surface's texture coordinate
+        const int lastMat = (int)(word & kStateMat);
+        uint32_t nextWord = 0u;
         const float t = h0.x;
         const int light = __float_as_int(h1.w);
         const int slot = __float_as_int(h0.w);
@@ -482,7 +416,7 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
             // material fetched is the last surface's (state is not refreshed),
             // its emission map read at that surface's texture coordinate
             Mat m = load_material(sc.materials, lastMat);
-            rad = rad + textured_emission(sc, lastMat, make_float2(misc.z, misc.w), m.emission) * thr;
+            rad = rad + textured_emission(sc, lastMat, texc, m.emission) * thr;
             V3 em = ld3(sc.lights[(size_t)light * kLightF4 + 1]);
             V3 Le = (depth == 0) ? em : powerHeuristic(prevPdf, h1.z) * em;
             rad = rad + Le * thr;
@@ -521,11 +455,14 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
             fr.N = dot(nrm, rd) <= 0.0f ? nrm : nrm * -1.0f;
             onb(nrm, fr.T, fr.B);
             fr.eta = dot(rd, nrm) < 0.0f ? (1.0f / m.ior) : m.ior;
-            V3 absorb = ld3(pb.absorb[p]);
-            if (dot(nrm, fr.N) > 0.0f) absorb = v3(0.f, 0.f, 0.f);
+            // a stored coefficient is not zero; a zero one multiplies by exactly 1
+            V3 absorb = v3(0.f, 0.f, 0.f);
             rad = rad + m.emission * thr;
-            lastMat = matId;
-            thr = thr * v3(expf(-absorb.x * t), expf(-absorb.y * t), expf(-absorb.z * t));
+            if ((word & kStateAbsorb) && !(dot(nrm, fr.N) > 0.0f)) {
+                absorb = ld3(pb.absorb[p]);
+                thr = thr * v3(expf(-absorb.x * t), expf(-absorb.y * t), expf(-absorb.z * t));
+            }
+            nextWord = (uint32_t)matId;
             uint4 rng = pb.rng[p];
             const float4* lob = gh.lobes + i;
             const size_t lst = (size_t)gh.lobe_stride;
@@ -578,10 +515,18 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
                     }
                 }
             }
-            if (shEnv || shLight) {
-                pb.nee[(size_t)p * 3 + 0] = e4;
-                pb.nee[(size_t)p * 3 + 1] = l4;
-                pb.nee[(size_t)p * 3 + 2] = f4(thr, 1.0f);
+            {
+                float4* nee = pb.nee + p;
+                if (shEnv && shLight) {
+                    nee[0] = e4;
+                    nee[pb.stride] = l4;
+                    nee[2 * pb.stride] = f4(thr, 1.0f);
+                } else if (shEnv) {
+                    nee[0] = f4(ld3(e4) * thr, 1.0f);
+                } else if (shLight) {
+                    nee[pb.stride] = f4(ld3(l4) * thr, 1.0f);
+                }
+                nextWord |= (shEnv ? kStateEnv : 0u) | (shLight ? kStateLight : 0u);
             }
             // BSDF sampling (pathtrace.glsl:268-291)
             V3 L;
@@ -636,24 +581,21 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
                 r[7] = luminance(thrBefore);
                 reinterpret_cast<float4*>(r)[3] = make_float4(L.x, L.y, L.z, 0.0f);
             }
-            pb.rng[p] = rng;
-            pb.thr[p] = f4(thr, 0.f);
-            pb.absorb[p] = f4(absorb, 0.f);
-            prevPdf = misPdf;
+            if (cont) {   // a path that ends here is shaded no more
+                pb.rng[p] = rng;
+                pb.thr[p] = f4(thr, misPdf);
+                if (!(absorb.x == 0.0f && absorb.y == 0.0f && absorb.z == 0.0f)) {
+                    pb.absorb[p] = f4(absorb, 0.f);
+                    nextWord |= kStateAbsorb;
+                }
+                if (sc.tex) pb.texc[p] = texc;
+            }
         }
-        pb.rad[p] = f4(rad, 0.f);
-        pb.misc[p] = make_float4(prevPdf, __int_as_float(lastMat), texc.x, texc.y);
+        pb.rad[p] = f4(rad, __uint_as_float(nextWord));
     }
-#if LFH_BLOCK_APPEND
-    __shared__ uint32_t app[16];
     uint32_t s = block_append(next_count, cont, app);
     uint32_t sl;
     uint32_t se = block_append2(shadow_count, shEnv, shLight, &sl, app);
-#else
-    uint32_t s = wave_append(next_count, cont);
-    uint32_t se = wave_append(shadow_count, shEnv);
-    uint32_t sl = wave_append(shadow_count, shLight);
-#endif
     if (cont) {
         nextq[(size_t)s * 2] = f4(nextO, __int_as_float(p));
         nextq[(size_t)s * 2 + 1] = f4(nextD, 0.f);
@@ -671,7 +613,7 @@ __global__ __launch_bounds__(256, LFH_SHADE_WAVES) void k_shade(ShadeScene sc1, 
 // ---- accumulate: pending NEE + Kahan sum into the frame -----------------------------
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_accumulate(PathBufs pb, int total, CamParams cam1, float4* accum1,
-                                                    float4* comp1, int kahan1, const JobDev* __restrict__ jobs) {
+                                                    float4* comp1, int kahan1, const JobDev* __restrict__ jobs, int keep) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= total) return;
     CamParams cam = cam1;
@@ -698,9 +640,10 @@ __global__ __launch_bounds__(256) void k_accumulate(PathBufs pb, int total, CamP
     const int P = cam.tile_w * cam.tile_h;
     for (int k = 0; k < nb; ++k) {
         const int q = p + k * P;
-        V3 rad = ld3(pb.rad[q]);
-        combine_nee(pb, q, rad);
-        pb.rad[q] = f4(rad, 0.f);   // final path radiance (guide training targets)
+        const float4 r4 = pb.rad[q];
+        V3 rad = ld3(r4);
+        combine_nee(pb, q, __float_as_uint(r4.w), rad);
+        if (keep) pb.rad[q] = f4(rad, 0.f);   // final path radiance (guide training targets)
         if (kahan) {
             float yx = rad.x - c.x, yy = rad.y - c.y, yz = rad.z - c.z;
             float tx = s.x + yx, ty = s.y + yy, tz = s.z + yz;
@@ -720,8 +663,9 @@ __global__ __launch_bounds__(256) void k_accumulate(PathBufs pb, int total, CamP
 __global__ void k_collect(PathBufs pb, int n, float* __restrict__ out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    V3 rad = ld3(pb.rad[p]);
-    combine_nee(pb, p, rad);
+    const float4 r4 = pb.rad[p];
+    V3 rad = ld3(r4);
+    combine_nee(pb, p, __float_as_uint(r4.w), rad);
     out[(size_t)p * 3] = rad.x;
     out[(size_t)p * 3 + 1] = rad.y;
     out[(size_t)p * 3 + 2] = rad.z;
@@ -846,24 +790,26 @@ hipError_t pt_reset(uint32_t* counters, unsigned long long* work, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t pt_generate(const CamParams& cam, const PathBufs& pb, float4* rayq, uint32_t* count, hipStream_t s) {
+hipError_t pt_generate(const CamParams& cam, int max_depth, const PathBufs& pb, float4* rayq, uint32_t* count,
+                       hipStream_t s) {
     int P = cam.tile_w * cam.tile_h * (cam.batch > 1 ? cam.batch : 1);
     hipLaunchKernelGGL(k_generate<false>, dim3(nblk(P)), dim3(256), 0, s, cam, (const JobDev*)nullptr, 1, P, pb, rayq,
-                       count);
+                       count, max_depth <= 0);
     return hipGetLastError();
 }
 
-hipError_t pt_generate_multi(const JobDev* jobs, int njobs, int total, const PathBufs& pb, float4* rayq,
+hipError_t pt_generate_multi(const JobDev* jobs, int njobs, int total, int max_depth, const PathBufs& pb, float4* rayq,
                              uint32_t* count, hipStream_t s) {
     CamParams dummy{};
     hipLaunchKernelGGL(k_generate<true>, dim3(nblk(total)), dim3(256), 0, s, dummy, jobs, njobs, total, pb, rayq,
-                       count);
+                       count, max_depth <= 0);
     return hipGetLastError();
 }
 
-hipError_t pt_generate_rays(const float* rays6, const uint4* seeds, int n, const PathBufs& pb, float4* rayq,
+hipError_t pt_generate_rays(const float* rays6, const uint4* seeds, int n, int max_depth, const PathBufs& pb, float4* rayq,
                             uint32_t* count, hipStream_t s) {
-    hipLaunchKernelGGL(k_generate_rays, dim3(nblk(n)), dim3(256), 0, s, rays6, seeds, n, pb, rayq, count);
+    hipLaunchKernelGGL(k_generate_rays, dim3(nblk(n)), dim3(256), 0, s, rays6, seeds, n, pb, rayq, count,
+                       max_depth <= 0);
     return hipGetLastError();
 }
 
@@ -912,18 +858,18 @@ hipError_t pt_bounces_multi(const JobDev* jobs, int max_depth, const PtQueues& q
     return bounces<true>(none, jobs, max_depth, q, pb, gh, gd, guide_sc ? *guide_sc : none, s);
 }
 
-hipError_t pt_accumulate_multi(const JobDev* jobs, int total, const PathBufs& pb, hipStream_t s) {
+hipError_t pt_accumulate_multi(const JobDev* jobs, int total, const PathBufs& pb, bool keep_radiance, hipStream_t s) {
     CamParams dummy{};
     hipLaunchKernelGGL(k_accumulate<true>, dim3(nblk(total)), dim3(256), 0, s, pb, total, dummy, (float4*)nullptr,
-                       (float4*)nullptr, 0, jobs);
+                       (float4*)nullptr, 0, jobs, keep_radiance ? 1 : 0);
     return hipGetLastError();
 }
 
 hipError_t pt_accumulate(const PathBufs& pb, const CamParams& cam, float4* accum, float4* comp, int kahan,
-                         hipStream_t s) {
+                         bool keep_radiance, hipStream_t s) {
     int P = cam.tile_w * cam.tile_h;
     hipLaunchKernelGGL(k_accumulate<false>, dim3(nblk(P)), dim3(256), 0, s, pb, P, cam, accum, comp, kahan,
-                       (const JobDev*)nullptr);
+                       (const JobDev*)nullptr, keep_radiance ? 1 : 0);
     return hipGetLastError();
 }
 

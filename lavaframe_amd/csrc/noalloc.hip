@@ -24,7 +24,7 @@
 namespace {
 
 constexpr int64_t kNoAllocPaths = (int64_t)1 << 16;   // paths per call, at most
-// per path: rad, thr, absorb, rng, misc (16 B each), nee (48), two ray queues
+// per path: rad, thr, absorb, rng, texc (16 B each), nee (48), two ray queues
 // (32 each), hit queue (32), shadow queue (64), job id (4)
 constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
@@ -99,8 +99,9 @@ extern "C" int lfh_path_trace_rays_device_noalloc(lfh_ctx* c, const float* d_ray
     pb.thr = reinterpret_cast<float4*>(take(kF4));
     pb.absorb = reinterpret_cast<float4*>(take(kF4));
     pb.rng = reinterpret_cast<uint4*>(take(kF4));
-    pb.misc = reinterpret_cast<float4*>(take(kF4));
+    pb.texc = reinterpret_cast<float2*>(take(kF4));
     pb.nee = reinterpret_cast<float4*>(take(3 * kF4));
+    pb.stride = kNoAllocPaths;
     PtQueues q;
     q.rayq[0] = reinterpret_cast<float4*>(take(2 * kF4));
     q.rayq[1] = reinterpret_cast<float4*>(take(2 * kF4));
@@ -117,7 +118,7 @@ extern "C" int lfh_path_trace_rays_device_noalloc(lfh_ctx* c, const float* d_ray
     if (off > kScratchBytes) return fail(c, LFH_E_INVALID, std::string(fn) + ": scratch layout exceeds its size");
     hipError_t e = pt_reset(q.counts, q.work, c->stream);   // counters start at zero (a kernel, no memset)
     if (e == hipSuccess)
-        e = pt_generate_rays(d_rays6, reinterpret_cast<const uint4*>(d_seeds), (int)n, pb, q.rayq[0], q.counts,
+        e = pt_generate_rays(d_rays6, reinterpret_cast<const uint4*>(d_seeds), (int)n, c->opt.max_depth, pb, q.rayq[0], q.counts,
                              c->stream);
     const lfhd::ShadeScene sc = lfh::shade_view(c->ps, c->ds, c->opt);
     if (e == hipSuccess) e = pt_bounces(sc, c->opt.max_depth, q, pb, GuideHook{}, nullptr, c->stream);

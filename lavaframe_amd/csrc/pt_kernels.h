@@ -6,15 +6,20 @@
 #include "dev_guide.h"
 #include "pt_types.h"
 
-// Path state, indexed by path id (tile pixel).
+// Path state, indexed by path id (tile pixel).  A path's first shading starts
+// it (generation writes only the random-number state), and a bounce reads and
+// writes what the path needs: absorb only inside an absorbing medium, texc
+// only in scenes with texture maps, the next-event arrays only for the terms a
+// vertex has.
 struct PathBufs {
-    float4* rad;     // radiance
-    float4* thr;     // throughput
+    float4* rad;     // radiance, state word (material, pending next-event terms, absorb stored)
+    float4* thr;     // throughput, previous BSDF pdf
     float4* absorb;  // Beer-Lambert absorption coefficient
     uint4* rng;      // pcg4d state
-    float4* misc;    // (previous BSDF pdf, last material id, 0, 0)
-    float4* nee;     // 3 per path: env term, light term (w = 1 while unoccluded), (throughput, pending)
+    float2* texc;    // last surface's texture coordinate
+    float4* nee;     // 3 arrays: env term, light term (w = 1 while unoccluded), throughput
     int* job;        // job id per path (multi-job passes only)
+    int64_t stride;  // paths per array of nee
 };
 
 // Learned-guide hook of a pass.
@@ -61,23 +66,27 @@ struct PtQueues {
 // Starts a wavefront: adds the ray counts the last one left to the totals and
 // clears the counters.
 hipError_t pt_reset(uint32_t* counters, unsigned long long* work, hipStream_t s);
-hipError_t pt_generate(const lfhd::CamParams& cam, const PathBufs& pb, float4* rayq, uint32_t* count, hipStream_t s);
-hipError_t pt_generate_rays(const float* rays6, const uint4* seeds, int n, const PathBufs& pb, float4* rayq,
+// max_depth: the depth of the bounces that follow
+hipError_t pt_generate(const lfhd::CamParams& cam, int max_depth, const PathBufs& pb, float4* rayq, uint32_t* count,
+                       hipStream_t s);
+hipError_t pt_generate_rays(const float* rays6, const uint4* seeds, int n, int max_depth, const PathBufs& pb, float4* rayq,
                             uint32_t* count, hipStream_t s);
 // All the bounces of a wavefront (gh.enabled: guided with gd's weights).
 hipError_t pt_bounces(const lfhd::ShadeScene& sc, int max_depth, const PtQueues& q, const PathBufs& pb,
                       const GuideHook& gh, const lfhd::GuideDev* gd, hipStream_t s);
 // Multi-job pass (serving): every job renders its full frame once; rays of all
 // jobs share the queues.  jobs: device table of njobs entries.
-hipError_t pt_generate_multi(const lfhd::JobDev* jobs, int njobs, int total, const PathBufs& pb, float4* rayq,
+hipError_t pt_generate_multi(const lfhd::JobDev* jobs, int njobs, int total, int max_depth, const PathBufs& pb, float4* rayq,
                              uint32_t* count, hipStream_t s);
 // gh.enabled: a guided wavefront, all of whose jobs render guide_sc's scene.
 hipError_t pt_bounces_multi(const lfhd::JobDev* jobs, int max_depth, const PtQueues& q, const PathBufs& pb,
                             const GuideHook& gh, const lfhd::GuideDev* gd, const lfhd::ShadeScene* guide_sc,
                             hipStream_t s);
-hipError_t pt_accumulate_multi(const lfhd::JobDev* jobs, int total, const PathBufs& pb, hipStream_t s);
+// keep_radiance: the paths' final radiance stays in pb.rad (guide training)
+hipError_t pt_accumulate_multi(const lfhd::JobDev* jobs, int total, const PathBufs& pb, bool keep_radiance,
+                               hipStream_t s);
 hipError_t pt_accumulate(const PathBufs& pb, const lfhd::CamParams& cam, float4* accum, float4* comp, int kahan,
-                         hipStream_t s);
+                         bool keep_radiance, hipStream_t s);
 hipError_t pt_collect(const PathBufs& pb, int n, float* out, hipStream_t s);
 hipError_t pt_output(const float4* accum, const float4* comp, int64_t npix, float inv, float* out, hipStream_t s);
 hipError_t pt_clear4(float4* a, int64_t n, hipStream_t s);

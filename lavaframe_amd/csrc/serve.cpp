@@ -544,7 +544,7 @@ static int run_group(lfh_server* s, const Group& g, const lfhd::JobDev* table_de
     uint32_t* cnt = pb.counters.as<uint32_t>();
     unsigned long long* work = pb.work.as<unsigned long long>();
     SCHK(s, pt_reset(cnt, work, s->stream), "lfh_server_step: reset");
-    SCHK(s, pt_generate_multi(table_dev, (int)g.jobs.size(), (int)total, v, pb.rq0.as<float4>(), cnt, s->stream),
+    SCHK(s, pt_generate_multi(table_dev, (int)g.jobs.size(), (int)total, max_depth, v, pb.rq0.as<float4>(), cnt, s->stream),
          "lfh_server_step: generate");
     GuideHook gh{};
     lfhd::GuideDev gd{};
@@ -577,7 +577,7 @@ static int run_group(lfh_server* s, const Group& g, const lfhd::JobDev* table_de
     } else {
         SCHK(s, chain(), "lfh_server_step: bounce");
     }
-    SCHK(s, pt_accumulate_multi(table_dev, (int)total, v, s->stream), "lfh_server_step: accumulate");
+    SCHK(s, pt_accumulate_multi(table_dev, (int)total, v, gh.train != 0, s->stream), "lfh_server_step: accumulate");
     if (g.guided_scene) {
         const int r = lfh::guide_end(ga, gh, batch);
         if (r != LFH_OK) return sfail(s, r, std::string("lfh_server_step: guide: ") + lfh_internal::thread_error());

@@ -386,3 +386,59 @@ def test_sphere_and_distant_lights_match_oracle():
         se = cr.std(0) / math.sqrt(m)
         assert np.all(np.abs(gr.mean(0) - cr.mean(0)) < 4 * se + 1e-6), est
         assert cr.mean() > 0.01
+
+
+@pytest.mark.parametrize("which", ["lights", "env", "both", "none", "media", "depth0", "depth1"])
+def test_path_state_kept_between_bounces(which):
+    """Each kind of path state a bounce may leave out: next-event terms of one
+    kind, of both, of none; absorption inside a medium and its absence; path
+    depth 0 (nothing is shaded) and 1.  Rays one by one through the renderer's
+    two layouts (lfh_path_trace_rays, the no-alloc entry point) and against the
+    oracle."""
+    import torch
+    print(f"[pt] path state {which}", flush=True)
+    s = lfh.Scene()
+    s.add_material(lfh.MATERIAL_DEFAULT)
+    glass = dict(transmission=1.0, ior=1.5, roughness=0.2)
+    if which == "media":
+        glass.update(extinction=(0.3, 0.6, 0.9), atDistance=0.5)
+    s.add_material(lfh.material((0.8, 0.7, 0.6), roughness=0.4))
+    s.add_material(lfh.material((0.9, 0.95, 0.9), **glass))
+    cube = s.add_mesh(scenes.unit_cube_tris())
+    s.add_instance(cube, scenes.affine(None, (8, 0.2, 8), (0, -1.0, 0)), 1)
+    s.add_instance(cube, scenes.affine(None, (0.8, 0.8, 0.8), (-0.5, 0, 0)), 2)
+    s.add_instance(cube, scenes.affine(None, (0.6, 0.9, 0.6), (0.6, 0, 0.3)), 1)
+    if which not in ("env", "none"):
+        s.add_light(lfh.quad_light((-1, 3, -1), (1, 3, -1), (-1, 3, 1), (6, 5, 4)))
+    if which not in ("lights", "none"):
+        s.set_hdr(scenes.sky_hdr(64, 32, sun_power=20.0))
+    s.set_camera((0, 1, 4), (0, 0, 0), 45)
+    depth = {"depth0": 0, "depth1": 1}.get(which, 6)
+    s.set_options(width=64, height=64, max_depth=depth, use_env_map=1 if which not in ("lights", "none") else 0,
+                  use_constant_bg=1 if which == "none" else 0, bg_color=(0.4, 0.5, 0.6), hdr_multiplier=1.0,
+                  enable_rr=1, rr_depth=2)
+    s.build()
+    ctx, arr = ctx_of(s), s.arrays()
+    rng = np.random.default_rng(7)
+    n = 30_011
+    rays = _camera_rays(s, n, rng)
+    seeds = rng.integers(0, 2**32, (n, 4), dtype=np.uint64).astype(np.uint32)
+    g = ctx.path_trace_rays(rays, seeds)
+    ctx.path_trace_rays(rays[::-1].copy(), seeds[::-1].copy())   # other state in the reused buffers
+    dr = torch.from_numpy(np.ascontiguousarray(rays, np.float32)).cuda()
+    ds = torch.from_numpy(seeds.view(np.int32)).cuda()
+    for _ in range(2):
+        out = torch.full((n, 3), -1.0, device="cuda")
+        torch.cuda.synchronize()
+        ctx._chk(ctx.lib.lfh_path_trace_rays_device_noalloc(ctx.h, dr.data_ptr(), ds.data_ptr(), n, out.data_ptr()))
+        ctx.synchronize()
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), g.view(np.uint32))
+    o = native.options_from(s.options(), s.camera(), lights=len(arr["lights"]) > 0,
+                            envmap=bool(s.options().use_env_map))
+    if depth:
+        c = native.OracleScene(arr).path_trace_rays(o, rays, seeds, 32)
+        same = np.isclose(g, c, rtol=1e-4, atol=1e-5).all(1)
+        assert same.mean() > 0.99, same.mean()
+        assert g.mean() > 0.01
+    else:
+        assert not g.any()
