@@ -74,30 +74,43 @@ LFH_DEV void sincos_pi(float v, float* s, float* c) {
 // sin a)(cos a + sin a), which multiply the base error by at most 2^5 at the
 // top octave: a few 1e-5 absolute, far below the BF16 step (2^-8 near 1) the
 // features are rounded to.
+// One axis: 12 features of the position, 4 of the normal, 4 of the outgoing
+// direction, each as sin, cos per octave.
+LFH_DEV void guide_encode_axis(float x, float n, float wo, float* f) {
+    float sn, cs;
+    sincos_pi(x, &sn, &cs);
+#pragma unroll
+    for (int fr = 0; fr < 6; ++fr) {
+        f[fr * 2] = sn;
+        f[fr * 2 + 1] = cs;
+        const float s2 = 2.0f * sn * cs, c2 = (cs - sn) * (cs + sn);
+        sn = s2;
+        cs = c2;
+    }
+    sincos_pi(n, &sn, &cs);
+    f[12] = sn;
+    f[13] = cs;
+    f[14] = 2.0f * sn * cs;
+    f[15] = (cs - sn) * (cs + sn);
+    sincos_pi(wo, &sn, &cs);
+    f[16] = sn;
+    f[17] = cs;
+    f[18] = 2.0f * sn * cs;
+    f[19] = (cs - sn) * (cs + sn);
+}
 LFH_DEV void guide_encode(V3 x, V3 n, V3 wo, float* f) {
     const float xs[3] = {x.x, x.y, x.z}, ns[3] = {n.x, n.y, n.z}, ws[3] = {wo.x, wo.y, wo.z};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float sn, cs;
-        sincos_pi(xs[a], &sn, &cs);
+        float v[20];
+        guide_encode_axis(xs[a], ns[a], ws[a], v);
 #pragma unroll
-        for (int fr = 0; fr < 6; ++fr) {
-            f[(a * 6 + fr) * 2] = sn;
-            f[(a * 6 + fr) * 2 + 1] = cs;
-            const float s2 = 2.0f * sn * cs, c2 = (cs - sn) * (cs + sn);
-            sn = s2;
-            cs = c2;
+        for (int k = 0; k < 12; ++k) f[a * 12 + k] = v[k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            f[36 + a * 4 + k] = v[12 + k];
+            f[48 + a * 4 + k] = v[16 + k];
         }
-        sincos_pi(ns[a], &sn, &cs);
-        f[36 + a * 4 + 0] = sn;
-        f[36 + a * 4 + 1] = cs;
-        f[36 + a * 4 + 2] = 2.0f * sn * cs;
-        f[36 + a * 4 + 3] = (cs - sn) * (cs + sn);
-        sincos_pi(ws[a], &sn, &cs);
-        f[48 + a * 4 + 0] = sn;
-        f[48 + a * 4 + 1] = cs;
-        f[48 + a * 4 + 2] = 2.0f * sn * cs;
-        f[48 + a * 4 + 3] = (cs - sn) * (cs + sn);
     }
     f[60] = wo.x;
     f[61] = wo.y;

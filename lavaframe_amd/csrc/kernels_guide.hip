@@ -360,12 +360,26 @@ __global__ void k_guide_pdf(const float4* __restrict__ lobes, const float* __res
 }
 
 // ---- training -----------------------------------------------------------------------
-// One block = 64 samples (4 waves x one 16-row tile).  Forward with the
-// activations kept in LDS, analytic d loss / d outputs per sample, then
-// backward: weight gradients dW = X^T dY (K = the block's samples) and
-// dX = (dY W^T) masked by ReLU, all as MFMA tiles.  Each block writes its
-// partial gradient; k_guide_reduce_adam sums the partials in block order, so
-// the result does not depend on scheduling.
+// One block = 64 samples (4 waves x one 16-row tile).  Forward, analytic
+// d loss / d outputs per sample, then backward: weight gradients dW = X^T dY
+// (K = the block's samples) and dX = (dY W^T) masked by ReLU, all as MFMA
+// tiles.  Each block writes its partial gradient; k_guide_reduce_adam sums the
+// partials in block order, so the result does not depend on scheduling.
+//
+// Bound by latency (2 waves per SIMD, a chain of 11 products) and by the partial
+// gradients, 60 KB per block.  Every operand is a 16 B LDS read: an MFMA result
+// holds four consecutive samples of one feature, so each layer's activations
+// and gradients are stored twice, feature-major for dW (one 8 B write per lane)
+// and row-major for the next layer's product, the latter in one buffer of 16
+// rows per wave, which no other wave reads.  Building dW's operands from
+// row-major rows took 512 two-byte LDS reads per lane.  A product's weights
+// come through LDS, fetched one product ahead with coalesced loads; reading
+// them as fragments from global memory, each wave its own, took 4700 cycles
+// per layer.  65536-sample step: 43 -> 28 us (107 -> 163 TFLOP/s in useful products;
+// the partials alone take about 12 us at the copy rate).
+// (Two tiles per block with their gradients added in registers halve the
+// partials' traffic, but change the order of the sums: a guide trained online
+// then ends elsewhere.)
 //
 // Samples: 4 float4 each: (pos, w), (n, 0), (wo, 0), (d, 0).
 struct TrainArgs {
@@ -392,95 +406,165 @@ LFH_DEV int batch_size(const TrainArgs& t) {
     return n > t.batch ? t.batch : n;
 }
 
-__global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideDev g, TrainArgs ta) {
-    __shared__ __attribute__((aligned(16))) uint16_t sA[4][kTrainRows * kPitch];  // E, H1, H2, H3
-    __shared__ __attribute__((aligned(16))) uint16_t sG0[kTrainRows * kPitch];
-    // the FP32 outputs (forward, loss) and the second gradient buffer
-    // (backward) are never live together
+// Orders this wave's LDS accesses: rows written by some lanes are read by others.
+LFH_DEV void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Features first .. first + 1 of sample s as a BF16 pair, in both layouts.
+LFH_DEV void put_pair(uint16_t* row, uint16_t* xt, int s, int first, float a, float b) {
+    const uint32_t v = pack_bf16x2(a, b);
+    *reinterpret_cast<uint32_t*>(row + first) = v;
+    xt[first * kPitch + s] = (uint16_t)v;
+    xt[(first + 1) * kPitch + s] = (uint16_t)(v >> 16);
+}
+
+__global__ __launch_bounds__(kTrainBlock, 2) void k_guide_train(GuideDev g, TrainArgs ta) {
+    __shared__ __attribute__((aligned(16))) uint16_t sXt[4][64 * kPitch];   // E, H1, H2, H3: [feature][sample]
+    __shared__ __attribute__((aligned(16))) uint16_t sRow[4][16 * kPitch];  // per wave: [sample][feature] of the current layer
+    __shared__ __attribute__((aligned(16))) uint16_t sGt0[64 * kPitch];     // dY [output][sample] of odd layers
+    // the FP32 outputs (forward, loss) and dY of even layers are never live together
     __shared__ __attribute__((aligned(16))) float sOG[kTrainRows * kOutPitch];
-    static_assert(sizeof(float) * kTrainRows * kOutPitch >= sizeof(uint16_t) * kTrainRows * kPitch, "alias size");
-    float* sO = sOG;
-    uint16_t* sG1 = reinterpret_cast<uint16_t*>(sOG);
+    static_assert(sizeof(float) * kTrainRows * kOutPitch >= sizeof(uint16_t) * 64 * kPitch, "alias size");
+    uint16_t* sGt1 = reinterpret_cast<uint16_t*>(sOG);
+    __shared__ __attribute__((aligned(16))) uint16_t sW[64 * kPitch];       // the current product's weights
     __shared__ float sD[kTrainRows][4];
     __shared__ float sLoss[kTrainRows];
     __shared__ float sDb[4][64];   // quarter sums of the bias gradient
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int lr = lane & 15, lk = (lane >> 4) * 8, lq = (lane >> 4) * 4;
+    const int lr = lane & 15, grp = lane >> 4, lk = grp * 8, lq = grp * 4;
     const int N = batch_size(ta);
     const int base = blockIdx.x * kTrainRows;
-    float* part = ta.partial + (size_t)blockIdx.x * kPartStride;
     if (base >= N) return;  // block-uniform; the reduction reads only active blocks
+    const int stride = batch_stride(ta), phase = batch_phase(ta);
+    float* part = ta.partial + (size_t)blockIdx.x * kPartStride;
+    uint16_t* row = sRow[wave];
+    const float invN = 1.0f / (float)N;
+    float wscale = 1.0f;
+    const bool weigh = ta.wsum != nullptr;
+    if (weigh) wscale = *ta.wsum / (float)*ta.count;   // the mean weight
 
-    // 1. encode: one thread per sample (rows past the batch are zero with w = 0)
-    if (tid < kTrainRows) {
-        const int s = tid;
+    // weights: 16 B chunks tid and tid + 256 of a [64][64] image, in registers
+    // while the product before uses sW
+    u32x4 wq0, wq1;
+    auto fetch_w = [&](const uint16_t* W) {
+        wq0 = reinterpret_cast<const u32x4*>(W)[tid];
+        wq1 = reinterpret_cast<const u32x4*>(W)[tid + 256];
+    };
+    auto put_w = [&]() {
+        uint16_t* p = sW + (tid >> 3) * kPitch + (tid & 7) * 8;
+        *reinterpret_cast<u32x4*>(p) = wq0;
+        *reinterpret_cast<u32x4*>(p + 32 * kPitch) = wq1;
+    };
+    // B fragment of columns 16 nt .. 16 nt + 15, K step ks
+    auto w_frag = [&](int nt, int ks) { return ld_frag(sW + (nt * 16 + lr) * kPitch + ks * 32 + lk); };
+    fetch_w(g.wf);
+
+    // 1. encode: lane s is sample s; waves 0..2 take an axis each, wave 3 the
+    // rest (rows past the batch are zero with w = 0)
+    {
+        const int s = lane;
         const bool ok = base + s < N;
-        uint16_t* row = sA[0] + s * kPitch;
+        uint16_t* r = sRow[s >> 4] + (s & 15) * kPitch;
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a, c = a;
         if (ok) {
-            const float4* sp = ta.samples + ((size_t)(base + s) * batch_stride(ta) + batch_phase(ta)) * 4;
-            const float4 a = sp[0], b = sp[1], c = sp[2], d = sp[3];
-            sD[s][0] = d.x;
-            sD[s][1] = d.y;
-            sD[s][2] = d.z;
-            float w = a.w;
-            if (ta.wsum) {
-                const float mean = *ta.wsum / (float)*ta.count;
-                w = mean > 0.0f ? fminf(w / mean, ta.wcap) : 0.0f;
+            const float4* sp = ta.samples + ((size_t)(base + s) * stride + phase) * 4;
+            a = sp[0];
+            if (wave < 3) b = sp[1];
+            c = sp[2];
+            if (wave == 3) {
+                const float4 d = sp[3];
+                float w = a.w;
+                if (weigh) w = wscale > 0.0f ? fminf(w / wscale, ta.wcap) : 0.0f;
+                sD[s][0] = d.x;
+                sD[s][1] = d.y;
+                sD[s][2] = d.z;
+                sD[s][3] = w;
             }
-            sD[s][3] = w;
-            encode_row(row, g, ld3(a), ld3(b), ld3(c));
-        } else {
+        } else if (wave == 3) {
             sD[s][0] = sD[s][1] = sD[s][2] = sD[s][3] = 0.0f;
-            for (int f = 0; f < kGuideIn; ++f) row[f] = 0;
+        }
+        const float on = ok ? 1.0f : 0.0f;
+        if (wave < 3) {
+            const float pa = wave == 0 ? a.x : (wave == 1 ? a.y : a.z);
+            const float na = wave == 0 ? b.x : (wave == 1 ? b.y : b.z);
+            const float wa = wave == 0 ? c.x : (wave == 1 ? c.y : c.z);
+            const float lo = wave == 0 ? g.lo[0] : (wave == 1 ? g.lo[1] : g.lo[2]);
+            const float ie = wave == 0 ? g.inv_ext[0] : (wave == 1 ? g.inv_ext[1] : g.inv_ext[2]);
+            float f[20];
+            guide_encode_axis(guide_norm_coord(pa, lo, ie), na, wa, f);
+#pragma unroll
+            for (int k = 0; k < 20; k += 2) {
+                const int first = k < 12 ? wave * 12 + k : (k < 16 ? 36 + wave * 4 + k - 12 : 48 + wave * 4 + k - 16);
+                put_pair(r, sXt[0], s, first, ok ? f[k] : 0.0f, ok ? f[k + 1] : 0.0f);
+            }
+        } else {
+            put_pair(r, sXt[0], s, 60, ok ? c.x : 0.0f, ok ? c.y : 0.0f);
+            put_pair(r, sXt[0], s, 62, ok ? c.z : 0.0f, on);
         }
     }
+    put_w();
     __syncthreads();
 
-    // 2. forward, wave w on rows 16w..16w+15; layer l reads sA[l], writes sA[l+1] (or sO)
+    // 2. forward, wave w on rows 16w..16w+15
 #pragma unroll
     for (int layer = 0; layer < kGuideLayers; ++layer) {
-        const uint16_t* W = g.wf + layer * 4096;
+        fetch_w(layer < 3 ? g.wf + (layer + 1) * 4096 : g.wb + 3 * 4096);
         const float* bias = g.bias + layer * 64;
         const int nN = layer == 3 ? 3 : 4;
-        const uint16_t* X = sA[layer];
+        const bf16x8 a0 = ld_frag(row + lr * kPitch + lk), a1 = ld_frag(row + lr * kPitch + 32 + lk);
         f32x4 acc[4];
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const bf16x8 a = ld_frag(X + (wave * 16 + lr) * kPitch + ks * 32 + lk);
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                if (nt < nN) acc[nt] = mfma(a, ld_frag(W + (nt * 16 + lr) * 64 + ks * 32 + lk), acc[nt]);
+        for (int nt = 0; nt < 4; ++nt) {
+            if (nt >= nN) continue;
+            acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[nt] = mfma(a0, w_frag(nt, 0), acc[nt]);
+            acc[nt] = mfma(a1, w_frag(nt, 1), acc[nt]);
         }
+        wave_lds_fence();
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
             if (nt >= nN) continue;
             const int col = nt * 16 + lr;
             const float b = bias[col];
+            if (layer < 3) {
+                const uint32_t lo = pack_bf16x2(fmaxf(acc[nt][0] + b, 0.0f), fmaxf(acc[nt][1] + b, 0.0f));
+                const uint32_t hi = pack_bf16x2(fmaxf(acc[nt][2] + b, 0.0f), fmaxf(acc[nt][3] + b, 0.0f));
+                *reinterpret_cast<uint2*>(sXt[layer + 1] + col * kPitch + wave * 16 + lq) = make_uint2(lo, hi);
+                row[(lq + 0) * kPitch + col] = (uint16_t)lo;
+                row[(lq + 1) * kPitch + col] = (uint16_t)(lo >> 16);
+                row[(lq + 2) * kPitch + col] = (uint16_t)hi;
+                row[(lq + 3) * kPitch + col] = (uint16_t)(hi >> 16);
+            } else if (col < kGuideOut) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int row = wave * 16 + lq + j;
-                const float v = acc[nt][j] + b;
-                if (layer < 3) sA[layer + 1][row * kPitch + col] = to_bf16(fmaxf(v, 0.0f));
-                else if (col < kGuideOut) sO[row * kOutPitch + col] = v;
+                for (int j = 0; j < 4; ++j) sOG[(wave * 16 + lq + j) * kOutPitch + col] = acc[nt][j] + b;
             }
         }
+        if (layer < 3) {
+            __syncthreads();   // every wave is done with sW
+            put_w();
+            __syncthreads();
+        } else {
+            wave_lds_fence();
+        }
     }
-    __syncthreads();
 
-    // 3. d loss / d outputs, BF16 into sG0 (cols 40..63 zero).  Four threads per
-    // sample, in one wave: sample 16 wave + lane % 16, lane group g = lane / 16
-    // takes lobes 2g and 2g+1; the softmax and log-sum-exp over the 8 lobes
-    // reduce over the 4 groups with shuffles (every group ends with the same
+    // 3. d loss / d outputs, BF16 in both layouts (outputs 40..63 zero).  Four
+    // threads per sample, in one wave: sample 16 wave + lane % 16, lane group g =
+    // lane / 16 takes lobes 2g and 2g+1; the softmax and log-sum-exp over the 8
+    // lobes reduce over the 4 groups with shuffles (every group ends with the same
     // sums: the two-step xor tree adds the same pairs in every lane).
-    const float invN = 1.0f / (float)N;
     {
-        const int s = wave * 16 + lr, grp = lane >> 4;
-        const float* o = sO + s * kOutPitch;
-        uint16_t* grow = sG0 + s * kPitch;
+        const int s = wave * 16 + lr;
+        const float* o = sOG + s * kOutPitch;
+        uint16_t* grow = row + lr * kPitch;
+        uint16_t* gt = sGt0 + s;
         const float w = sD[s][3];
-        for (int c = kGuideOut + grp * 6; c < kGuideOut + grp * 6 + 6; ++c) grow[c] = 0;
+        for (int c = kGuideOut + grp * 6; c < kGuideOut + grp * 6 + 6; ++c) {
+            grow[c] = 0;
+            gt[c * kPitch] = 0;
+        }
         const V3 d = v3(sD[s][0], sD[s][1], sD[s][2]);
         const int k0 = 2 * grp;
         float amax = fmaxf(o[5 * k0 + 4], o[5 * k0 + 9]);
@@ -515,6 +599,7 @@ __global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideDev g, TrainAr
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int k = k0 + j;
+            float gv[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
             if (w != 0.0f) {
                 const float gam = expf(lw[j] - lmax) / gs;
                 const float e2 = expf(-2.0f * kap[j]);
@@ -522,18 +607,23 @@ __global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideDev g, TrainAr
                 const float sraw = o[5 * k + 3];
                 const bool inside = sraw > kLogKMin && sraw < kLogKMax;
                 const float gr = -sc * gam * kap[j] / rn[j];
-                grow[5 * k + 0] = to_bf16(gr * (d.x - cs[j] * mu[j].x));
-                grow[5 * k + 1] = to_bf16(gr * (d.y - cs[j] * mu[j].y));
-                grow[5 * k + 2] = to_bf16(gr * (d.z - cs[j] * mu[j].z));
-                grow[5 * k + 3] = to_bf16(inside ? -sc * gam * kap[j] * dlogv : 0.0f);
-                grow[5 * k + 4] = to_bf16(sc * (pi[j] - gam));
-            } else {
+                gv[0] = gr * (d.x - cs[j] * mu[j].x);
+                gv[1] = gr * (d.y - cs[j] * mu[j].y);
+                gv[2] = gr * (d.z - cs[j] * mu[j].z);
+                gv[3] = inside ? -sc * gam * kap[j] * dlogv : 0.0f;
+                gv[4] = sc * (pi[j] - gam);
+            }
 #pragma unroll
-                for (int c = 0; c < 5; ++c) grow[5 * k + c] = 0;
+            for (int c = 0; c < 5; ++c) {
+                const uint16_t h = to_bf16(gv[c]);
+                grow[5 * k + c] = h;
+                gt[(5 * k + c) * kPitch] = h;
             }
         }
         if (grp == 0) sLoss[s] = w != 0.0f ? -w * (lmax + logf(gs)) * invN : 0.0f;
     }
+    __syncthreads();
+    put_w();           // layer 3's backward weights
     __syncthreads();
     if (tid < 64) {
         float l = sLoss[tid];
@@ -541,80 +631,82 @@ __global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideDev g, TrainAr
         if (tid == 0) part[kGuideParams] = l;
     }
 
-    // 4. backward, layers 3..0.  dY of layer l is in (l odd ? sG0 : sG1) — l = 3: sG0.
+    // 4. backward, layers 3..0.  dY of layer l: row-major in the wave's rows,
+    // output-major in sGt0 (l odd) or sGt1.
 #pragma unroll
     for (int layer = 3; layer >= 0; --layer) {
-        uint16_t* dY = (layer & 1) ? sG0 : sG1;
-        uint16_t* dX = (layer & 1) ? sG1 : sG0;
-        const uint16_t* X = sA[layer];
-        const int nout = guide_layer_out(layer);
-        const int off = guide_layer_offset(layer);
-        // dW[i][o] = sum_s X[s][i] dY[s][o]: wave w computes in-tile it = w for every out tile
+        if (layer > 1) fetch_w(g.wb + (layer - 1) * 4096);   // the next product's weights
+        const uint16_t* dYt = (layer & 1) ? sGt0 : sGt1;
+        uint16_t* dXt = (layer & 1) ? sGt1 : sGt0;
+        const uint16_t* Xt = sXt[layer];
+        const int nout = guide_layer_out(layer), off = guide_layer_offset(layer);
+        // dW[i][o] = sum_s X[s][i] dY[s][o]: wave w takes in-tile w for every out tile
         {
-            const int it = wave;
+            const bf16x8 a0 = ld_frag(Xt + (wave * 16 + lr) * kPitch + lk),
+                         a1 = ld_frag(Xt + (wave * 16 + lr) * kPitch + 32 + lk);
             const int nOt = layer == 3 ? 3 : 4;
 #pragma unroll
             for (int ot = 0; ot < 4; ++ot) {
                 if (ot >= nOt) continue;
-                f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    bf16x8 a, b;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int s = ks * 32 + lk + j;
-                        uint16_t xa = X[s * kPitch + it * 16 + lr];
-                        uint16_t yb = dY[s * kPitch + ot * 16 + lr];
-                        a[j] = __builtin_bit_cast(__bf16, xa);
-                        b[j] = __builtin_bit_cast(__bf16, yb);
-                    }
-                    acc = mfma(a, b, acc);
-                }
+                f32x4 dw = f32x4{0.f, 0.f, 0.f, 0.f};
+                dw = mfma(a0, ld_frag(dYt + (ot * 16 + lr) * kPitch + lk), dw);
+                dw = mfma(a1, ld_frag(dYt + (ot * 16 + lr) * kPitch + 32 + lk), dw);
                 const int col = ot * 16 + lr;
                 if (col < nout) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int in = it * 16 + lq + j;
-                        part[off + in * nout + col] = acc[j];
-                    }
+                    for (int j = 0; j < 4; ++j) part[off + (wave * 16 + lq + j) * nout + col] = dw[j];
                 }
             }
         }
-        // db[o] = sum_s dY[s][o]: four quarter sums of 16 rows per output,
-        // then added in quarter order
+        // db[o] = sum_s dY[s][o]: four quarter sums of 16 rows per output, then added
+        // in quarter order
         {
-            const int o = tid & 63, q = tid >> 6;
+            const uint16_t* y = dYt + (tid & 63) * kPitch + (tid >> 6) * 16;
+            const u32x4 y0 = *reinterpret_cast<const u32x4*>(y), y1 = *reinterpret_cast<const u32x4*>(y + 8);
             float sum = 0.0f;
 #pragma unroll
-            for (int s = 0; s < kTrainRows / 4; ++s) sum += from_bf16(dY[(q * (kTrainRows / 4) + s) * kPitch + o]);
-            sDb[q][o] = sum;
+            for (int k = 0; k < 4; ++k) {
+                sum += from_bf16((uint16_t)y0[k]);
+                sum += from_bf16((uint16_t)(y0[k] >> 16));
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                sum += from_bf16((uint16_t)y1[k]);
+                sum += from_bf16((uint16_t)(y1[k] >> 16));
+            }
+            sDb[tid >> 6][tid & 63] = sum;
         }
-        __syncthreads();
-        if (tid < nout) part[off + 64 * nout + tid] = ((sDb[0][tid] + sDb[1][tid]) + sDb[2][tid]) + sDb[3][tid];
         if (layer > 0) {
             // dX[s][i] = (sum_o dY[s][o] W[i][o]) * (X[s][i] > 0), rows of this wave
-            const uint16_t* WB = g.wb + layer * 4096;
+            const bf16x8 a0 = ld_frag(row + lr * kPitch + lk), a1 = ld_frag(row + lr * kPitch + 32 + lk);
             f32x4 acc[4];
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const bf16x8 a = ld_frag(dY + (wave * 16 + lr) * kPitch + ks * 32 + lk);
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt) acc[nt] = mfma(a, ld_frag(WB + (nt * 16 + lr) * 64 + ks * 32 + lk), acc[nt]);
+            for (int nt = 0; nt < 4; ++nt) {
+                acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                acc[nt] = mfma(a0, w_frag(nt, 0), acc[nt]);
+                acc[nt] = mfma(a1, w_frag(nt, 1), acc[nt]);
             }
+            wave_lds_fence();
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) {
                 const int col = nt * 16 + lr;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int row = wave * 16 + lq + j;
-                    const bool on = from_bf16(X[row * kPitch + col]) > 0.0f;
-                    dX[row * kPitch + col] = to_bf16(on ? acc[nt][j] : 0.0f);
-                }
+                const uint2 x = *reinterpret_cast<const uint2*>(Xt + col * kPitch + wave * 16 + lq);
+                const float v0 = from_bf16((uint16_t)x.x) > 0.0f ? acc[nt][0] : 0.0f;
+                const float v1 = from_bf16((uint16_t)(x.x >> 16)) > 0.0f ? acc[nt][1] : 0.0f;
+                const float v2 = from_bf16((uint16_t)x.y) > 0.0f ? acc[nt][2] : 0.0f;
+                const float v3 = from_bf16((uint16_t)(x.y >> 16)) > 0.0f ? acc[nt][3] : 0.0f;
+                const uint32_t lo = pack_bf16x2(v0, v1), hi = pack_bf16x2(v2, v3);
+                *reinterpret_cast<uint2*>(dXt + col * kPitch + wave * 16 + lq) = make_uint2(lo, hi);
+                row[(lq + 0) * kPitch + col] = (uint16_t)lo;
+                row[(lq + 1) * kPitch + col] = (uint16_t)(lo >> 16);
+                row[(lq + 2) * kPitch + col] = (uint16_t)hi;
+                row[(lq + 3) * kPitch + col] = (uint16_t)(hi >> 16);
             }
         }
-        __syncthreads();
+        __syncthreads();   // dXt and sDb are whole; every wave is done with dYt and sW
+        if (tid < nout) part[off + 64 * nout + tid] = ((sDb[0][tid] + sDb[1][tid]) + sDb[2][tid]) + sDb[3][tid];
+        if (layer > 1) put_w();
+        if (layer > 0) __syncthreads();
     }
 }
 
@@ -637,8 +729,7 @@ constexpr int kReduceChunks = 32;
 __global__ void k_guide_reduce1(TrainArgs ta, float* __restrict__ chunks) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j > kGuideParams) return;
-    const int N = batch_size(ta);
-    const int nb = (N + kTrainRows - 1) / kTrainRows;
+    const int nb = (batch_size(ta) + kTrainRows - 1) / kTrainRows;
     const int per = (nb + kReduceChunks - 1) / kReduceChunks;
     const int b0 = blockIdx.y * per, b1 = min(nb, b0 + per);
     float sum = 0.0f;
@@ -653,8 +744,7 @@ __global__ void k_guide_reduce_adam(TrainArgs ta, AdamArgs ad, const float* __re
                                     float* __restrict__ grad_out, float* __restrict__ loss_out) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j > kGuideParams) return;
-    const int N = batch_size(ta);
-    const int nb = (N + kTrainRows - 1) / kTrainRows;
+    const int nb = (batch_size(ta) + kTrainRows - 1) / kTrainRows;
     float sum = 0.0f;
     for (int r = 0; r < kReduceChunks; ++r) sum += chunks[(size_t)r * kPartStride + j];
     if (j == kGuideParams) {
@@ -753,8 +843,16 @@ __global__ __launch_bounds__(1024) void k_guide_scan(CollectArgs c, int nblocks)
     const int t = threadIdx.x;
     const int per = (nblocks + 1023) / 1024;
     const int b0 = t * per;
+    const int b1 = min(b0 + per, nblocks);
+    // eight counts in flight: one block works through up to 40960 of them
     int local = 0;
-    for (int b = b0; b < b0 + per && b < nblocks; ++b) local += c.block_counts[b];
+    for (int b = b0; b < b1; b += 8) {
+        int n[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) n[k] = b + k < b1 ? c.block_counts[b + k] : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) local += n[k];
+    }
     s[t] = local;
     __syncthreads();
     for (int off = 1; off < 1024; off <<= 1) {
@@ -765,10 +863,21 @@ __global__ __launch_bounds__(1024) void k_guide_scan(CollectArgs c, int nblocks)
     }
     int run = s[t] - local;
     float wl = 0.0f;
-    for (int b = b0; b < b0 + per && b < nblocks; ++b) {
-        c.block_offsets[b] = run;
-        if (run + c.block_counts[b] <= c.max_samples) wl += c.block_wsum[b];
-        run += c.block_counts[b];
+    for (int b = b0; b < b1; b += 8) {
+        int n[8];
+        float w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            n[k] = b + k < b1 ? c.block_counts[b + k] : 0;
+            w[k] = b + k < b1 ? c.block_wsum[b + k] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (b + k >= b1) break;
+            c.block_offsets[b + k] = run;
+            if (run + n[k] <= c.max_samples) wl += w[k];
+            run += n[k];
+        }
     }
     sws[t] = wl;
     __syncthreads();

@@ -151,6 +151,28 @@ def test_loss_and_gradient_match_oracle():
         assert np.linalg.norm(grad[o:o + n_] - r) < 0.08 * np.linalg.norm(r) + 1e-9, l
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 129, 65535])
+def test_loss_and_gradient_at_tile_edges(n):
+    """Batches that end inside a wave's 16-row tile, a block's 64 samples or
+    exactly on their edges (rows past the batch must add nothing).  Same bounds
+    as above: BF16 operands carry 2^-9 relative per product, a few of them in a
+    chain, so a few percent for a single sample too."""
+    print(f"[guide] loss / grad n={n}", flush=True)
+    g, p = _guide(seed=6, scale=0.15)
+    q, d, w = _batch(n, 30 + n)
+    w[0] = 1.0
+    loss, grad = g.loss_grad(q, d, w)
+    enc = _enc(q)
+    ref, rl = G.loss_grad(p, enc, d, w), G.loss(p, enc, d, w)
+    assert abs(loss - rl) < 1e-2 * max(1.0, abs(rl)), (loss, rl)
+    for l in range(4):
+        o, n_ = G.layer_slice(l)
+        r = ref[o:o + n_]
+        assert np.linalg.norm(grad[o:o + n_] - r) < 0.08 * np.linalg.norm(r) + 1e-9, l
+    l2, g2 = g.loss_grad(q, d, w)
+    assert l2 == loss and np.array_equal(g2, grad)
+
+
 def test_adam_first_step_closed_form():
     print("[guide] adam", flush=True)
     g, p0 = _guide(seed=7)
