@@ -137,15 +137,26 @@ bool bounce_graphs_enabled() {
 // Reads (and clears) the overflow flag the path-tracing passes set when a
 // traversal stack overflowed; the accumulation is then incomplete.  The
 // scene's stack need is checked at lfh_create, so this is a safety net.
-int check_render_flag(lfh_ctx* c) {
-    int flag = 0;
-    RCHK(c, hipMemcpyAsync(&flag, c->rflag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream), "render flag");
-    RCHK(c, hipStreamSynchronize(c->stream), "render flag");
+static int render_flag_result(lfh_ctx* c, int flag) {
     if (flag) {
         RCHK(c, pt_clear_flag(c->rflag.as<int>(), c->stream), "render flag");
         return rfail(c, LFH_E_UNSUPPORTED, "traversal stack overflow while rendering (image incomplete)");
     }
     return LFH_OK;
+}
+
+int check_render_flag(lfh_ctx* c) {
+    int flag = 0;
+    RCHK(c, hipMemcpyAsync(&flag, c->rflag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream), "render flag");
+    RCHK(c, hipStreamSynchronize(c->stream), "render flag");
+    return render_flag_result(c, flag);
+}
+
+// Copies the output staging buffer to the caller and checks the flag, with one wait.
+static int read_output(lfh_ctx* c, void* dst, size_t bytes, const char* fn) {
+    int flag = 0;
+    RCHK(c, c->readback.read(dst, c->out.p, bytes, c->rflag.as<int>(), &flag, c->device, c->stream), fn);
+    return render_flag_result(c, flag);
 }
 
 // Paths per wavefront targeted by multi-sample passes over one-tile frames
@@ -317,7 +328,8 @@ int lfh_render_preview(lfh_ctx* c, float scale, int32_t use_dof, float* dst, int
         RCHK(c, pt_output(c->preview.as<float4>(), c->preview.as<float4>() + n, n, 1.0f, c->out.as<float>(),
                           c->stream),
              "lfh_render_preview: output");
-        RCHK(c, hipMemcpyAsync(dst, c->out.p, bytes, hipMemcpyDeviceToHost, c->stream), "lfh_render_preview: copy");
+        RCHK(c, c->readback.read(dst, c->out.p, bytes, nullptr, nullptr, c->device, c->stream), "lfh_render_preview: copy");
+        return LFH_OK;
     }
     RCHK(c, hipStreamSynchronize(c->stream), "lfh_render_preview: sync");
     return LFH_OK;
@@ -423,9 +435,7 @@ int lfh_get_output_hdr(lfh_ctx* c, float* dst, int32_t w, int32_t h) {
     float inv = 1.0f / (float)c->sampleCounter;
     RCHK(c, pt_output(c->rs.accum.as<float4>(), c->rs.comp.as<float4>(), c->rs.npix, inv, c->out.as<float>(), c->stream),
          "lfh_get_output_hdr: kernel");
-    RCHK(c, hipMemcpyAsync(dst, c->out.p, bytes, hipMemcpyDeviceToHost, c->stream), "lfh_get_output_hdr: copy");
-    RCHK(c, hipStreamSynchronize(c->stream), "lfh_get_output_hdr: sync");
-    return lfh::check_render_flag(c);
+    return lfh::read_output(c, dst, bytes, "lfh_get_output_hdr: copy");
 }
 
 static int get_post(lfh_ctx* c, const lfh_postprocess* pp, float inv, float* rgb, uint8_t* ldr, int32_t w,
@@ -452,9 +462,7 @@ static int get_post(lfh_ctx* c, const lfh_postprocess* pp, float inv, float* rgb
     RCHK(c, lfhd::post_process(c->rs.accum.as<float4>(), c->rs.comp.as<float4>(), w, h, inv, p,
                                rgb ? c->out.as<float>() : nullptr, rgb ? nullptr : c->out.as<uint8_t>(), c->stream),
          fn);
-    RCHK(c, hipMemcpyAsync(rgb ? (void*)rgb : (void*)ldr, c->out.p, bytes, hipMemcpyDeviceToHost, c->stream), fn);
-    RCHK(c, hipStreamSynchronize(c->stream), fn);
-    return lfh::check_render_flag(c);
+    return lfh::read_output(c, rgb ? (void*)rgb : (void*)ldr, bytes, fn);
 }
 
 int lfh_get_output_post(lfh_ctx* c, const lfh_postprocess* pp, float inv, float* dst, int32_t w, int32_t h) {

@@ -10,6 +10,7 @@
 #include "dev_common.h"
 #include "pt_kernels.h"
 #include "pt_types.h"
+#include "readback.h"
 
 namespace lfh {
 
@@ -257,6 +258,7 @@ struct lfh_ctx {
     lfh::RenderState rs;
     lfh::PassBufs pass;
     lfh::DevBuf out;   // HDR output staging
+    lfh::Readback readback;
     int pt_grid = 0;
     lfh_camera cam{};
     bool has_cam = false;

@@ -1,0 +1,105 @@
+#include "readback.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+
+namespace lfh {
+
+void Readback::release() {
+    for (hipEvent_t& e : ev_) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    cap_ = 0;
+}
+
+hipError_t Readback::ensure(size_t bytes) {
+    const size_t want = std::min((size_t)kPieces, (bytes + kPiece - 1) / kPiece) * kPiece;
+    if (cap_ >= want) return hipSuccess;
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    cap_ = 0;
+    void* p = nullptr;
+    hipError_t e = hipHostMalloc(&p, want + 64, hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    pin_ = static_cast<char*>(p);
+    cap_ = want;
+    for (hipEvent_t& v : ev_)
+        if (e == hipSuccess && !v) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    if (e != hipSuccess) release();
+    return e;
+}
+
+hipError_t Readback::read(void* dst, const void* src, size_t bytes, const int* d_flag, int* flag, int device,
+                          hipStream_t s) {
+    // less than a piece and no flag to fetch along: the runtime's staging is as fast
+    // (six served images of 84-691 kB: 0.08 ms less in all)
+    const bool plain = bytes < kPiece && !d_flag;
+    if (plain || ensure(bytes) != hipSuccess) {
+        if (!plain) (void)hipGetLastError();   // no pinned memory to be had
+        hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess && d_flag) e = hipMemcpyAsync(flag, d_flag, sizeof(int), hipMemcpyDeviceToHost, s);
+        const hipError_t w = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : w;
+    }
+    if (d_flag) {
+        hipError_t e = hipMemcpyAsync(pin_ + cap_, d_flag, sizeof(int), hipMemcpyDeviceToHost, s);
+        if (e != hipSuccess) return e;
+    }
+    for (size_t w0 = 0; w0 < bytes; w0 += cap_) {   // windows of the pinned buffer
+        const size_t wn = std::min(cap_, bytes - w0);
+        const int n = (int)((wn + kPiece - 1) / kPiece);
+        hipError_t e = hipSuccess;
+        int queued = 0;
+        for (; queued < n; ++queued) {
+            const size_t o = (size_t)queued * kPiece;
+            e = hipMemcpyAsync(pin_ + o, static_cast<const char*>(src) + w0 + o, std::min(kPiece, wn - o),
+                               hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(ev_[queued], s);
+            if (e != hipSuccess) break;
+        }
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s);   // nothing may still write the pinned buffer
+            return e;
+        }
+        std::atomic<int> next{0};
+        std::atomic<int> err{(int)hipSuccess};
+        auto take = [&]() {
+            for (int k = next.fetch_add(1); k < n; k = next.fetch_add(1)) {
+                const hipError_t r = hipEventSynchronize(ev_[k]);
+                if (r != hipSuccess) {
+                    err.store((int)r);
+                    return;
+                }
+                const size_t o = (size_t)k * kPiece;
+                std::memcpy(static_cast<char*>(dst) + w0 + o, pin_ + o, std::min(kPiece, wn - o));
+            }
+        };
+        std::thread pool[kThreads - 1];
+        const int extra = std::min(n, kThreads) - 1;
+        for (int t = 0; t < extra; ++t) {
+            try {
+                pool[t] = std::thread([&] {
+                    if (hipSetDevice(device) == hipSuccess) take();
+                });
+            } catch (...) {
+                break;   // fewer helpers; this thread takes what is left
+            }
+        }
+        take();
+        for (std::thread& t : pool)
+            if (t.joinable()) t.join();
+        if (err.load() != (int)hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            return (hipError_t)err.load();
+        }
+    }
+    if (d_flag) std::memcpy(flag, pin_ + cap_, sizeof(int));   // copied before the first piece
+    return hipSuccess;
+}
+
+}  // namespace lfh

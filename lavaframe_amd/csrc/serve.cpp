@@ -252,6 +252,9 @@ struct lfh_server {
     lfh::BounceGraph bgraph;               // the plain group's bounce chain
     int64_t gbuf_charged = 0;
     lfh::DevBuf table, spill, errflag;
+    lfh::DevBuf out;                       // lfh_server_result's image
+    lfh::Readback readback;
+    int device = 0;
     int grid = 0;
     int64_t used = 0;  // resident scenes + accum of admitted jobs + path shares of running jobs
     std::string err;
@@ -358,7 +361,8 @@ int lfh_server_create(int64_t budget_bytes, int32_t max_jobs, lfh_server** out) 
         budget_bytes = (int64_t)(0.9 * (double)f);
     }
     s->budget = budget_bytes;
-    hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
+    hipError_t e = hipGetDevice(&s->device);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->upload_stream, hipStreamNonBlocking);
     if (e == hipSuccess) {
         s->grid = pt_trace_grid_blocks();
@@ -403,6 +407,8 @@ void lfh_server_destroy(lfh_server* s) {
     s->table.release();
     s->spill.release();
     s->errflag.release();
+    s->out.release();
+    s->readback.release();
     if (s->upload_stream) hipStreamDestroy(s->upload_stream);
     if (s->stream) hipStreamDestroy(s->stream);
     delete s;
@@ -862,13 +868,13 @@ int lfh_server_result(lfh_server* s, int64_t id, float* dst, int32_t w, int32_t 
     lfh::Job& j = *it->second;
     if (j.state != 2 && j.state != 1) return sfail(s, LFH_E_STATE, "lfh_server_result: job has no samples");
     if (w != j.opt.width || h != j.opt.height) return sfail(s, LFH_E_INVALID, "lfh_server_result: size mismatch");
-    DevBuf out;
-    SCHK(s, out.alloc((size_t)j.npix * 12), "lfh_server_result: alloc");
+    const size_t bytes = (size_t)j.npix * 12;
+    if (s->out.bytes < bytes) SCHK(s, s->out.alloc(bytes), "lfh_server_result: alloc");
     SCHK(s, pt_output(j.accum.as<float4>(), j.comp.as<float4>(), j.npix, 1.0f / (float)std::max(1, j.spp_done),
-                      out.as<float>(), s->stream),
+                      s->out.as<float>(), s->stream),
          "lfh_server_result: kernel");
-    SCHK(s, hipMemcpyAsync(dst, out.p, (size_t)j.npix * 12, hipMemcpyDeviceToHost, s->stream), "lfh_server_result: copy");
-    SCHK(s, hipStreamSynchronize(s->stream), "lfh_server_result: sync");
+    SCHK(s, s->readback.read(dst, s->out.p, bytes, nullptr, nullptr, s->device, s->stream),
+         "lfh_server_result: copy");
     return LFH_OK;
 }
 

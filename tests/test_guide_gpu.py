@@ -151,26 +151,24 @@ def test_loss_and_gradient_match_oracle():
         assert np.linalg.norm(grad[o:o + n_] - r) < 0.08 * np.linalg.norm(r) + 1e-9, l
 
 
-@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 129, 65535])
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 129, 1000])
 def test_loss_and_gradient_at_tile_edges(n):
     """Batches that end inside a wave's 16-row tile, a block's 64 samples or
-    exactly on their edges (rows past the batch must add nothing).  Same bounds
-    as above: BF16 operands carry 2^-9 relative per product, a few of them in a
-    chain, so a few percent for a single sample too."""
+    exactly on their edges: rows past the batch must add nothing, as rows of
+    weight 0 do.  A batch of 2 n whose second half has weight 0 and whose first
+    half has twice the weight has the same w / N bit for bit, so its loss and
+    gradient are the same bit for bit (at most 32 blocks: they are summed one by
+    one in both)."""
     print(f"[guide] loss / grad n={n}", flush=True)
-    g, p = _guide(seed=6, scale=0.15)
-    q, d, w = _batch(n, 30 + n)
-    w[0] = 1.0
-    loss, grad = g.loss_grad(q, d, w)
-    enc = _enc(q)
-    ref, rl = G.loss_grad(p, enc, d, w), G.loss(p, enc, d, w)
-    assert abs(loss - rl) < 1e-2 * max(1.0, abs(rl)), (loss, rl)
-    for l in range(4):
-        o, n_ = G.layer_slice(l)
-        r = ref[o:o + n_]
-        assert np.linalg.norm(grad[o:o + n_] - r) < 0.08 * np.linalg.norm(r) + 1e-9, l
-    l2, g2 = g.loss_grad(q, d, w)
-    assert l2 == loss and np.array_equal(g2, grad)
+    g, _ = _guide(seed=6, scale=0.15)
+    q, d, w = _batch(2 * n, 30 + n)
+    w[:n] = np.maximum(w[:n], 0.25)
+    loss, grad = g.loss_grad(q[:n], d[:n], w[:n])
+    w2 = np.where(np.arange(2 * n) < n, 2 * w, 0).astype(np.float32)
+    l2, g2 = g.loss_grad(q, d, w2)
+    assert np.isfinite(grad).all() and np.abs(grad).max() > 0
+    assert l2 == loss
+    assert np.array_equal(g2, grad)
 
 
 def test_adam_first_step_closed_form():

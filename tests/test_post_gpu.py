@@ -64,3 +64,22 @@ def test_default_sample_count():
     ctx.render_passes(4)
     pp = lfh.Postprocess.make(tonemap_index=0)
     np.testing.assert_array_equal(ctx.output_post(pp), ctx.output_hdr())
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (349, 251), (512, 171), (1024, 1024), (3000, 1001)])
+def test_images_of_any_size_come_back_whole(w, h):
+    """Images of less than a MiB, just around one, and of more MiB than the
+    pinned staging holds at once (36 MB of floats): the float read-back equals
+    the raw sum scaled on the host, on a first and on a repeated call."""
+    print(f"[post] read-back {w}x{h}", flush=True)
+    sc = scenes.cornell(w, h, max_depth=2)
+    ctx = lfh.Context.from_scene(sc)
+    ctx.update(sc.camera(), reset=True)
+    ctx.render_passes(1)
+    s, c = ctx.accum()
+    want = (s - c) * np.float32(1.0 / ctx.sample_count())
+    for _ in range(2):
+        assert np.array_equal(ctx.output_hdr().view(np.uint32), want.view(np.uint32))
+    ldr = ctx.output_ldr(lfh.Postprocess.make())
+    assert np.array_equal(ldr, ctx.output_ldr(lfh.Postprocess.make())) and (w * h < 1000 or ldr.any())
+    assert np.array_equal(ctx.output_hdr().view(np.uint32), want.view(np.uint32))
