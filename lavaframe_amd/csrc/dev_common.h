@@ -69,9 +69,9 @@ LFH_HD uint32_t make_inst(uint32_t inst) { return kRefInstBit | inst; }
 // Work counters of the persistent traversal kernels: a queue's ray ids are
 // split into kFetchSlices contiguous slices, each with its own counter
 // kFetchStride 64-bit words (256 B) from the next.  A wavefront keeps
-// kQueueSets sets of queue counters in turn, depth d using set d % kQueueSets:
-// the ray counts (extension, shadow) and both queues' fetch counters; two
-// running ray totals follow the fetch counters at kWorkTotals.
+// kQueueSets sets of queue counters in turn, traversal d using set
+// d % kQueueSets: the ray counts (extension, shadow) and both queues' fetch
+// counters; two running ray totals follow the fetch counters at kWorkTotals.
 #ifndef LFH_FETCH_SLICES
 #define LFH_FETCH_SLICES 8
 #endif

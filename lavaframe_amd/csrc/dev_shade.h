@@ -533,6 +533,16 @@ LFH_DEV void camera_ray(const CamParams& c, int lx, int ly, V3& org, V3& dir, ui
     V3 focalPoint = c.focal_dist * rayDir;
     float cam_r1 = rnd(seed) * kTwoPi;
     float cam_r2 = rnd(seed) * c.aperture;
+    // a pinhole's lens offset is +-0, which changes nothing but the sign of a zero: of any
+    // zero it is subtracted from, of a negative zero it is added to
+    const bool zeros = focalPoint.x == 0.0f || focalPoint.y == 0.0f || focalPoint.z == 0.0f ||
+                       __float_as_uint(pos.x) == 0x80000000u || __float_as_uint(pos.y) == 0x80000000u ||
+                       __float_as_uint(pos.z) == 0x80000000u;
+    if (c.aperture == 0.0f && !zeros) {
+        dir = normalize(focalPoint);
+        org = pos;
+        return;
+    }
     V3 ap = (cosf(cam_r1) * right + sinf(cam_r1) * up) * sqrtf(cam_r2);
     dir = normalize(focalPoint - ap);
     org = pos + ap;

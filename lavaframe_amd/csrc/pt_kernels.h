@@ -47,9 +47,9 @@ struct GuideHook {
 using lfhd::GuideHook;
 
 
-// Queues and counters of a wavefront.  counts: (extension, shadow) rays of
-// each of the kQueueSets counter sets; work: their fetch counters and the
-// running ray totals.
+// Queues and counters of a wavefront.  counts: the (extension, shadow) rays
+// that each of kQueueSets traversals in turn takes, 8-byte aligned pairs;
+// work: their fetch counters and the running ray totals.
 struct PtQueues {
     float4* rayq[2];      // extension rays of even and odd depths, 2 float4 each
     float4* hitq;         // 2 float4 per extension ray
