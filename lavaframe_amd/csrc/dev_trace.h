@@ -76,7 +76,11 @@ struct LaneStack {
 // slice once exhausted stays so, and every id below n is handed out exactly
 // once.
 #ifndef LFH_FETCH_CHUNK
-#define LFH_FETCH_CHUNK 64
+// 64 / 128 / 192 / 256: 16.8M-ray closest hit 5.95 / 5.59 / 5.44 / 5.41 ms, 2M-ray any hit 765 / 749 / 781 / 787 us,
+// 8.4M incoherent rays 3.50 / 3.52 / 3.57 / 3.58 ms, C0 2.41 / 2.31 / 2.33 / 2.32 ms, viewer 720p 9.52 / 9.31 / 9.42 /
+// 9.52 ms, served mix 4.68 / 4.56 / 4.61 / 4.65 ms: longer chunks save atomics, and leave the waves that end a queue
+// with more rays each
+#define LFH_FETCH_CHUNK 128
 #endif
 #ifndef LFH_FETCH_MIN
 // 1021 rays, 20k triangles: at least 1 / 4 / 16 / 64 rays per wave 71 / 97 / 115 / 110 us (159 us with

@@ -11,8 +11,8 @@ from oracle import native
 
 pytestmark = pytest.mark.gpu
 
-# 256 CUs x 5 or 6 blocks x 4 waves x 64 rays: the largest queues without dynamic fetches
-CLOSEST, ANY = 256 * 5 * 4 * 64, 256 * 6 * 4 * 64
+# 256 CUs x 5 or 6 blocks x 4 waves x 128 rays: the largest queues without dynamic fetches
+CLOSEST, ANY = 256 * 5 * 4 * 128, 256 * 6 * 4 * 128
 
 
 @pytest.fixture(scope="module")
