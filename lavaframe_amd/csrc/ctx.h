@@ -195,7 +195,7 @@ struct GuideBufs {
     int nslots = 0;                // record slots: recorded paths x max_depth, largest wavefront
 };
 
-// The per-depth launch chain of a wavefront (trace, shade, shadow, advance for
+// The per-depth launch chain of a wavefront (trace, shade for
 // every depth) captured once as a HIP graph and replayed: its kernels read the
 // queue counters on the device, so the chain is the same for every wavefront
 // of one path capacity, scene, job table and depth.  `key` lists what the

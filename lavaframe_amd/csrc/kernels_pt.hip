@@ -324,7 +324,7 @@ LFH_DEV void trace_queue(const ShadeScene& sc, const JobDev* __restrict__ jobs, 
 // rays go to the waves in reverse order, so that in small wavefronts other
 // waves take them.
 #ifndef LFH_QUEUE_WAVES
-#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD: 6 / 5: C0 3.10 / 3.26 ms, instanced 1080p frame 22.3 / 24.4 ms
+#define LFH_QUEUE_WAVES 6   // queue traversal register budget, waves per SIMD: 7 / 6 / 5: C0 2.84 / 2.41 / 2.39 ms, instanced 1080p frame 22.6 / 19.0 / 19.8 ms, guiding room 7.43 / 6.25 / 6.39 ms, textured tiles 4.53 / 4.13 / 3.93 ms
 #endif
 template <bool MULTI>
 __global__ __launch_bounds__(kTraceBlock, LFH_QUEUE_WAVES) void k_trace_queues(ShadeScene sc, const JobDev* __restrict__ jobs,
