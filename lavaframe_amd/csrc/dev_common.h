@@ -140,7 +140,9 @@ LFH_DEV uint32_t as_u(float f) { return __float_as_uint(f); }
 // at a distance t0 <= lim, infinity for any other box.  min/max are IEEE
 // minNum/maxNum.  Both lower limits go into max(t0, the least positive float),
 // for closest hit both upper ones into min(t1, lim), so one comparison
-// decides (two for any hit).
+// decides (two for any hit).  min(t1, lim) also asks for a positive lim, so for
+// closest hit lim is at least the least positive float: at best distance 0 a
+// box around the origin still passes.
 //
 // The key decides how many nodes a ray visits, not what it hits:
 //   closest hit  t0, also where it is negative: of the boxes around the origin

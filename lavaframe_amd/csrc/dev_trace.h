@@ -340,7 +340,9 @@ template <bool ANY, bool STATS>
 LFH_DEV uint32_t visit_node(const NodeRec& nd, bool plain, TraceState& s, LaneStack& st, float cull,
                             TraceStats* stats) {
     if (STATS) stats->nint++;
-    const float lim = s.tbest * cull;
+    // a closest hit at distance 0 (a ray from a mesh vertex) leaves the boxes around the origin
+    // open: the triangle its tie goes to may be in one of them
+    const float lim = ANY ? s.tbest * cull : fmaxf(s.tbest * cull, kLeastPositive);
     const float none = __builtin_inff();
     float h[4];      // order key of a hit child, infinity otherwise
     uint32_t r[4] = {as_u(nd.rf.x), as_u(nd.rf.y), as_u(nd.rf.z), as_u(nd.rf.w)};

@@ -151,3 +151,76 @@ def test_rays_leaving_flat_walls_match_oracle(device_bvh):
     gh = ctx.trace_closest(rays)
     _compare(gh, orc.trace_closest(rays, tie_mode=1))
     assert not (gh["t"][gh["prim"] >= 0] <= 0).any()
+
+
+def _hits_at_zero(v, org, d):
+    """For every ray, the lowest triangle of v it hits at exactly t = 0 (-1:
+    none) and whether it leaves that triangle's own box at a positive
+    distance; every triangle tested, in the kernels' FP32 operations."""
+    v0, e0, e1 = v[:, 0], v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]
+    lo, hi = v.min(1), v.max(1)
+
+    def cross(a, b):
+        return np.stack([a[..., 1] * b[..., 2] - a[..., 2] * b[..., 1], a[..., 2] * b[..., 0] - a[..., 0] * b[..., 2],
+                         a[..., 0] * b[..., 1] - a[..., 1] * b[..., 0]], -1)
+
+    def dot(a, b):
+        p = a * b
+        return (p[..., 0] + p[..., 1]) + p[..., 2]
+
+    tri = np.full(len(org), -1)
+    inside = np.zeros(len(org), bool)
+    with np.errstate(all="ignore"):
+        for i in range(len(org)):
+            pv = cross(d[i], e1)
+            tv = org[i] - v0
+            qv = cross(tv, e0)
+            det = dot(e0, pv)
+            u, w, t = dot(tv, pv) / det, dot(np.broadcast_to(d[i], qv.shape), qv) / det, dot(e1, qv) / det
+            k = np.nonzero((u >= 0) & (w >= 0) & (t == 0) & (1 - u - w >= 0))[0]
+            if k.size:
+                tri[i] = k[0]
+                inside[i] = ((np.where(d[i] > 0, hi[k[0]], lo[k[0]]) - org[i]) / d[i]).min() > 0
+    return tri, inside
+
+
+@pytest.mark.parametrize("device_bvh", [False, True])
+def test_ties_at_distance_zero_go_to_the_lowest_triangle(device_bvh):
+    """Rays that start on a mesh vertex hit every triangle around it at t = 0
+    (and its copies: some triangles are there twice, the mesh in two
+    instances).  The lowest (instance, prim) whose own box the ray enters (it
+    leaves that box at a positive distance, the AABBIntersect > 0 rule) is in
+    open boxes of every tree, so both trees must find it."""
+    print(f"[trace] ties at 0 device_bvh={device_bvh}", flush=True)
+    rng = np.random.default_rng(17)
+    m = 33
+    g = np.stack(np.meshgrid(np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 2) / (m - 1.0)
+    p = np.concatenate([g, rng.uniform(0, 0.05, (len(g), 1))], 1)
+    q, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+    p = (p @ q).astype(np.float32)
+    c = (np.arange(m - 1)[:, None] * m + np.arange(m - 1)).reshape(-1)
+    ids = np.concatenate([np.stack([c, c + m, c + 1], 1), np.stack([c + m + 1, c + 1, c + m], 1)])
+    ids = rng.permutation(ids)
+    ids = np.concatenate([ids, ids[::5]])
+    tris = p[ids]
+    s = lfh.Scene()
+    s.add_material(lfh.MATERIAL_DEFAULT)
+    mesh = s.add_mesh(tris)
+    s.add_instance(mesh, None, 0)
+    s.add_instance(mesh, None, 0)
+    s.build()
+    n = 3000
+    r = scenes.incoherent_rays(n, seed=19)
+    r["org"] = p[rng.integers(0, len(p), n)]
+    want, inside = _hits_at_zero(tris, r["org"], r["dir"])
+    at0 = (want >= 0) & inside
+    assert at0.sum() > 400
+    ctx = lfh.Context.from_scene(s, device_bvh=device_bvh)
+    got, orc = ctx.trace_closest(r), native.OracleScene(s.arrays()).trace_closest(r, tie_mode=1)
+    assert np.array_equal(orc["prim"][at0], want[at0])
+    bad = got["prim"][at0] != want[at0]
+    assert not bad.any(), f"{bad.sum()} of {at0.sum()} rays"
+    assert not got["inst"][at0].any()
+    for f in ("t", "u", "v"):
+        assert np.array_equal(got[f][at0].view(np.uint32), orc[f][at0].view(np.uint32)), f
+    assert np.array_equal(ctx.trace_any(r).astype(bool), got["prim"] >= 0)
