@@ -118,7 +118,8 @@ __global__ void k_pt_reset(uint32_t* counts, unsigned long long* work) {
 }
 
 // generate: one thread per tile pixel (MULTI: per pixel of every job).
-// unshaded: no depth will be shaded (path depth 0), so the radiance starts here.
+// unshaded: no depth will be shaded (path depth 0), so the radiance starts here and
+// no ray is queued: nothing would trace it, and a queue's count goes to the ray totals.
 // whole: every path has a pixel (tiles inside the frame), so path p's ray goes to
 // slot p.  Tiles that stick out of the frame append their rays, one atomic per
 // block; on whole frames those bound the kernel (4.2M paths 194 -> 59 us,
@@ -162,6 +163,7 @@ __global__ __launch_bounds__(256) void k_generate(CamParams cam1, const JobDev* 
         pb.rng[p] = seed;
         if (unshaded) pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    if (unshaded) return;   // of the whole launch
     uint32_t slot = (uint32_t)p;
     if (whole) {
         if (p == 0) *count = (uint32_t)total;
@@ -185,6 +187,7 @@ __global__ __launch_bounds__(256) void k_generate_rays(const float* __restrict__
         pb.rng[p] = seeds[p];
         if (unshaded) pb.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    if (unshaded) return;   // as in k_generate
     if (p == 0) *count = (uint32_t)n;
     if (valid) {
         const float* r = rays6 + (size_t)p * 6;

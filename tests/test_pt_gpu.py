@@ -442,3 +442,33 @@ def test_path_state_kept_between_bounces(which):
         assert g.mean() > 0.01
     else:
         assert not g.any()
+
+
+@pytest.mark.parametrize("tile", [0, 24])
+def test_ray_counts_hold_the_rays_that_were_traced(tile):
+    """lfh_get_ray_counts over frames of whole tiles and of tiles that stick
+    out of the frame (40 x 24 tiles of 24): one extension ray per pixel and
+    pass at depth 1, at least that many and at most depth times as many
+    deeper, none at depth 0, where no ray is traced; asking does not change
+    the counts."""
+    print(f"[pt] ray counts tile={tile}", flush=True)
+    for depth in (0, 1, 2, 5):
+        sc = scenes.cornell(40, 24, max_depth=depth)
+        if tile:
+            sc.set_options(width=40, height=24, max_depth=depth, tile_width=tile, tile_height=tile)
+        ctx = ctx_of(sc)
+        ctx.update(sc.camera(), reset=True)
+        passes = 4
+        for _ in range(passes):
+            ctx.update(sc.camera())
+            ctx.render()
+        tiles = 1 if not tile else 2
+        pixels = 40 * 24 * passes // tiles   # tiles of 24 and 16 columns in turn
+        ext, shadow = ctx.ray_counts()
+        assert (ext, shadow) == ctx.ray_counts()
+        if depth == 0:
+            assert (ext, shadow) == (0, 0)
+        elif depth == 1:
+            assert ext == pixels and 0 < shadow <= ext
+        else:
+            assert pixels < ext <= depth * pixels and 0 < shadow <= ext
