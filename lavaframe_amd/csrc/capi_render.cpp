@@ -109,7 +109,7 @@ int render_init(lfh_ctx* c) {
     if (e == hipSuccess) e = c->rs.comp.alloc(npix * sizeof(float4));
     if (e == hipSuccess) e = pt_clear4(c->rs.accum.as<float4>(), npix, c->stream);
     if (e == hipSuccess) e = pt_clear4(c->rs.comp.as<float4>(), npix, c->stream);
-    if (e == hipSuccess) e = c->pass.alloc(c->rs.npaths);
+    if (e == hipSuccess) e = c->pass.alloc(c->rs.npaths, c->stream);
     if (e == hipSuccess) e = c->rflag.alloc(64);
     if (e == hipSuccess) e = hipMemsetAsync(c->rflag.p, 0, 64, c->stream);
     if (e == hipSuccess) {
@@ -199,7 +199,7 @@ int render_tile(lfh_ctx* c, int batch) {
         const int64_t need = (int64_t)c->rs.npaths * (batch > 1 ? batch : 1);
         if (c->pass.cap < need) {
             hipError_t e = hipStreamSynchronize(c->stream);
-            if (e == hipSuccess) e = c->pass.alloc((int)need);
+            if (e == hipSuccess) e = c->pass.alloc((int)need, c->stream);
             if (e != hipSuccess) return rhip(c, e, "render: path buffers");
         }
     }
@@ -264,7 +264,7 @@ int render_preview(lfh_ctx* c, float scale, int dof, int* pw, int* ph) {
     const int64_t n = (int64_t)W * H;
     if (c->pass.cap < n) {
         hipError_t e = hipStreamSynchronize(c->stream);
-        if (e == hipSuccess) e = c->pass.alloc((int)n);
+        if (e == hipSuccess) e = c->pass.alloc((int)n, c->stream);
         if (e != hipSuccess) return rhip(c, e, "lfh_render_preview: buffers");
     }
     // the frame, then a zero compensation buffer for the readback kernel
@@ -620,7 +620,7 @@ int lfh_path_trace_rays(lfh_ctx* c, const float* rays6, uint32_t* seeds, int64_t
     if (const char* m = stage_check(c, n)) return rfail(c, LFH_E_INVALID, std::string(fn) + ": " + m);
     if (n == 0) return LFH_OK;
     lfh::PassBufs pb;
-    RCHK(c, pb.alloc((int)n), fn);
+    RCHK(c, pb.alloc((int)n, c->stream), fn);
     Tmp tmp;
     hipError_t e;
     TMP(dr, float, n * 6) TMP(ds, uint4, n) TMP(dout, float, n * 3)

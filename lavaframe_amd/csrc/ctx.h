@@ -147,10 +147,12 @@ struct PassBufs {
     int cap = 0;
     // All or nothing: on any failure every buffer is released and cap is 0,
     // so the next caller that needs paths allocates again instead of
-    // launching on a half-allocated set.
-    hipError_t alloc(int n) {
+    // launching on a half-allocated set.  The counters are cleared on `s`, the
+    // stream of the passes: a wavefront starts from what they hold, and the
+    // null stream is not ordered with a non-blocking one.
+    hipError_t alloc(int n, hipStream_t s) {
         release();
-        hipError_t e = alloc_all(n);
+        hipError_t e = alloc_all(n, s);
         if (e != hipSuccess) {
             release();
             return e;
@@ -169,7 +171,7 @@ struct PassBufs {
     }
 
 private:
-    hipError_t alloc_all(int n) {
+    hipError_t alloc_all(int n, hipStream_t s) {
         if (lfh_internal::inject_fault(lfh_internal::kFaultPathAlloc)) return hipErrorOutOfMemory;
         hipError_t e;
         const size_t f4 = 16;
@@ -179,8 +181,8 @@ private:
             if ((e = b[i]->alloc(f4 * m[i] * (size_t)n)) != hipSuccess) return e;
         if ((e = counters.alloc(64)) != hipSuccess) return e;
         if ((e = work.alloc(lfhd::kWorkWords * 8)) != hipSuccess) return e;
-        if ((e = hipMemset(counters.p, 0, 64)) != hipSuccess) return e;
-        if ((e = hipMemset(work.p, 0, lfhd::kWorkWords * 8)) != hipSuccess) return e;
+        if ((e = hipMemsetAsync(counters.p, 0, 64, s)) != hipSuccess) return e;
+        if ((e = hipMemsetAsync(work.p, 0, lfhd::kWorkWords * 8, s)) != hipSuccess) return e;
         if ((e = job.alloc(4 * (size_t)n)) != hipSuccess) return e;
         return hipSuccess;
     }

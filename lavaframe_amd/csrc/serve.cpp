@@ -788,7 +788,7 @@ int lfh_server_step(lfh_server* s, int32_t* active) {
                 // grow with headroom, shrink only when far too large (a reallocation waits for the GPU)
                 const int64_t pcap = std::min<int64_t>(largest + largest / 4, std::max<int64_t>(largest, lfh::kStepPaths));
                 SCHK(s, hipStreamSynchronize(s->stream), "lfh_server_step: sync");
-                SCHK(s, s->pass.alloc((int)pcap), "lfh_server_step: path buffers");
+                SCHK(s, s->pass.alloc((int)pcap, s->stream), "lfh_server_step: path buffers");
             }
             const bool any_guided = groups.size() > 1;
             if (any_guided) {

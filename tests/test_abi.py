@@ -2,6 +2,7 @@
 rejects bad input with status codes and messages (no GPU needed: every case
 here fails before any device work)."""
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -20,6 +21,18 @@ def test_exports_every_declared_symbol(lib):
 def test_native_library_is_in_tree():
     assert lfh.LIB_PATH.exists()
     assert lfh.LIB_PATH.parent.parent.name == "lavaframe_amd"
+
+
+def test_device_clears_name_their_stream():
+    """Contexts and servers work on non-blocking streams, which the null stream
+    is not ordered with: a clear queued on the null stream could land after
+    the first kernel that counts on it (or writes what it clears)."""
+    csrc = lfh.LIB_PATH.parent.parent / "csrc"
+    files = [f for f in csrc.iterdir() if f.suffix in (".cpp", ".hip", ".h")]
+    assert len(files) > 20
+    on_null = [f"{f.name}: {line.strip()}" for f in files for line in f.read_text().splitlines()
+               if re.search(r"\bhipMemset(D8|D16|D32|2D|3D)?\(", line)]
+    assert on_null == []
 
 
 def test_null_arguments_return_invalid(lib):

@@ -472,3 +472,16 @@ def test_ray_counts_hold_the_rays_that_were_traced(tile):
             assert ext == pixels and 0 < shadow <= ext
         else:
             assert pixels < ext <= depth * pixels and 0 < shadow <= ext
+
+
+def test_ray_counts_start_at_zero_with_new_path_buffers():
+    """Path buffers that grow are cleared before the first wavefront counts on
+    them: at depth 1 every growth leaves exactly the rays of its own passes."""
+    print("[pt] ray counts after growth", flush=True)
+    for _ in range(3):
+        sc = scenes.cornell(64, 64, max_depth=1)
+        ctx = ctx_of(sc)
+        ctx.update(sc.camera(), reset=True)
+        for passes in (2, 5, 11, 23, 47):
+            ctx.render_passes(passes)
+            assert ctx.ray_counts()[0] == 64 * 64 * passes
