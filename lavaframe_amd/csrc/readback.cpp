@@ -66,6 +66,13 @@ hipError_t Readback::read(void* dst, const void* src, size_t bytes, const int* d
             (void)hipStreamSynchronize(s);   // nothing may still write the pinned buffer
             return e;
         }
+        // The copies may stand behind a frame: one thread waits for the first piece,
+        // and only then do others join it.
+        e = hipEventSynchronize(ev_[0]);
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            return e;
+        }
         std::atomic<int> next{0};
         std::atomic<int> err{(int)hipSuccess};
         auto take = [&]() {
