@@ -34,11 +34,22 @@ hipError_t Readback::ensure(size_t bytes) {
     return e;
 }
 
+// Memory the runtime knows (pinned, managed), which it transfers to without staging.
+static bool known_to_runtime(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 hipError_t Readback::read(void* dst, const void* src, size_t bytes, const int* d_flag, int* flag, int device,
                           hipStream_t s) {
-    // less than a piece and no flag to fetch along: the runtime's staging is as fast
-    // (six served images of 84-691 kB: 0.08 ms less in all)
-    const bool plain = bytes < kPiece && !d_flag;
+    // pinned memory of the caller: one transfer, no CPU copy (1080p 847 -> 485 us,
+    // 720p 391 -> 234 us); less than a piece and no flag to fetch along: the runtime's
+    // staging is as fast (six served images of 84-691 kB: 0.08 ms less in all)
+    const bool plain = (bytes < kPiece && !d_flag) || known_to_runtime(dst);
     if (plain || ensure(bytes) != hipSuccess) {
         if (!plain) (void)hipGetLastError();   // no pinned memory to be had
         hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);

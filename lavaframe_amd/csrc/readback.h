@@ -1,4 +1,4 @@
-// Device results to caller memory through pinned staging.
+// Device results to caller memory, through pinned staging where that is pageable.
 //
 // A copy to pageable memory goes through the runtime's own staging buffer one
 // MiB at a time, the transfer and the CPU copy (which also faults in the

@@ -14,6 +14,10 @@
 
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorUnknown = 999 };
 enum hipMemcpyKind { hipMemcpyDeviceToHost = 2 };
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t {
+    hipMemoryType type;
+};
 enum { hipHostMallocDefault = 0, hipEventDisableTiming = 2 };
 using hipStream_t = int;
 
@@ -27,6 +31,8 @@ inline int helpers = 0;                  // threads that set their device
 inline int waiting = 0, most_waiting = 0;   // threads in hipEventSynchronize while the gate was closed
 inline bool no_pinned = false;           // hipHostMalloc fails
 inline int fail_copy = -1, fail_sync = -1;   // the n-th copy / event wait from now fails
+inline const void* known = nullptr;      // the caller's pinned memory
+inline int copies = 0;
 inline int pinned = 0, events = 0;       // allocated and not yet given back
 
 inline void work() {
@@ -110,6 +116,7 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) {
 }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     if (fake::counted_down(fake::fail_copy)) return hipErrorUnknown;
+    fake::copies++;
     fake::push([=] { std::memcpy(d, s, n); });
     return hipSuccess;
 }
@@ -121,6 +128,10 @@ inline hipError_t hipStreamSynchronize(hipStream_t) {
 inline hipError_t hipSetDevice(int) {
     std::lock_guard<std::mutex> lk(fake::mu);
     fake::helpers++;
+    return hipSuccess;
+}
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    a->type = p == fake::known ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
     return hipSuccess;
 }
 inline hipError_t hipGetLastError() { return hipSuccess; }

@@ -78,6 +78,15 @@ int main() {
         CHECK(r == hipSuccess && flag == 5 && dst == src);
         CHECK(fake::helpers == 3);
 
+        begin("pinned memory of the caller: one transfer and the flag's, no helpers");
+        fake::known = dst.data();
+        fake::copies = fake::helpers = 0;
+        std::fill(dst.begin(), dst.end(), (unsigned char)0);
+        flag = 0;
+        CHECK(rb.read(dst.data(), src.data(), src.size(), &d_flag, &flag, 0, 0) == hipSuccess);
+        CHECK(flag == 5 && dst == src && fake::copies == 2 && fake::helpers == 0);
+        fake::known = nullptr;
+
         begin("a failed copy or wait is reported and leaves nothing behind");
         for (int k = 0; k < 12; ++k) {
             fake::fail_copy = k;

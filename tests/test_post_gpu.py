@@ -12,6 +12,8 @@ compares them where the rounding is not amplified:
 * Chromatic aberration reads at computed texture coordinates.  A float32
   coordinate is off by up to W 2^-24 ~ 4e-6 texel, times the texel contrast at
   a light's edge, so those cases allow 1e-4 relative."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -83,3 +85,21 @@ def test_images_of_any_size_come_back_whole(w, h):
     ldr = ctx.output_ldr(lfh.Postprocess.make())
     assert np.array_equal(ldr, ctx.output_ldr(lfh.Postprocess.make())) and (w * h < 1000 or ldr.any())
     assert np.array_equal(ctx.output_hdr().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("w,h", [(64, 48), (1000, 701)])
+def test_images_into_pinned_memory(w, h):
+    """Images read into the caller's pinned memory equal those read into
+    ordinary memory."""
+    import torch
+    print(f"[post] pinned {w}x{h}", flush=True)
+    sc = scenes.cornell(w, h, max_depth=2)
+    ctx = lfh.Context.from_scene(sc)
+    ctx.update(sc.camera(), reset=True)
+    ctx.render_passes(1)
+    want = ctx.output_hdr()
+    pin = torch.full((h, w, 3), -1.0).pin_memory()
+    for _ in range(2):
+        ctx._chk(ctx.lib.lfh_get_output_hdr(ctx.h, C.cast(pin.data_ptr(), lfh.f32p), w, h))
+        assert np.array_equal(pin.numpy().view(np.uint32), want.view(np.uint32))
+        pin.fill_(-1.0)
