@@ -364,7 +364,11 @@ typedef struct lfh_job_status {
     int64_t device_bytes;
 } lfh_job_status;
 
-/* budget_bytes: device memory the server may hold across jobs (0 = 90% of free).
+/* budget_bytes: device memory the server may hold across jobs (0 = 90% of free):
+ * scenes, accumulation buffers, path state, guide buffers and the image buffer
+ * of lfh_server_result.  Beside it the server holds its traversal stacks and
+ * job table, about 0.2 GB whatever the jobs, and at most 32 MiB of pinned host
+ * memory for results.
  * max_jobs: concurrent job slots (<= 64). */
 int  lfh_server_create(int64_t budget_bytes, int32_t max_jobs, lfh_server** out);
 void lfh_server_destroy(lfh_server* srv);

@@ -252,11 +252,11 @@ struct lfh_server {
     lfh::BounceGraph bgraph;               // the plain group's bounce chain
     int64_t gbuf_charged = 0;
     lfh::DevBuf table, spill, errflag;
-    lfh::DevBuf out;                       // lfh_server_result's image
-    lfh::Readback readback;
+    lfh::DevBuf out;                       // lfh_server_result's image (kept while the budget has room, in `used`; under mu)
+    lfh::Readback readback;                // under mu
     int device = 0;
     int grid = 0;
-    int64_t used = 0;  // resident scenes + accum of admitted jobs + path shares of running jobs
+    int64_t used = 0;  // resident scenes + accum of admitted jobs + path shares of running jobs + the kept image
     std::string err;
     // admission thread: uploads scenes queued by the step loop
     std::mutex mu;
@@ -289,9 +289,16 @@ static int shipfail(lfh_server* s, hipError_t e, const char* where) {
         if (_e != hipSuccess) return shipfail(s, _e, where);  \
     } while (0)
 
-// Evict unreferenced resident scenes (oldest first) until `need` more bytes
-// fit.  Called with the server mutex held.
+// Gives back the kept image buffer.  Called with the server mutex held.
+static void drop_image(lfh_server* s) {
+    s->used -= (int64_t)s->out.bytes;
+    s->out.release();
+}
+
+// Drops the kept image buffer, then evicts unreferenced resident scenes (oldest
+// first) until `need` more bytes fit.  Called with the server mutex held.
 static void evict_for(lfh_server* s, int64_t need) {
+    if (s->used + need > s->budget) drop_image(s);
     while (s->used + need > s->budget) {
         std::shared_ptr<lfh::SceneEntry> victim;
         for (auto& kv : s->scenes) {
@@ -682,6 +689,11 @@ int lfh_server_step(lfh_server* s, int32_t* active) {
     if (!running.empty()) {
         int64_t one_pass = 0;
         for (lfh::Job* j : running) one_pass += j->npix;
+        {
+            // a step's paths come before the kept image
+            std::lock_guard<std::mutex> lk(s->mu);
+            if (s->budget - s->used < lfh::kStepPaths * lfh::kPathBytes) drop_image(s);
+        }
         const int64_t spare = std::max<int64_t>(0, (s->budget - s->used) / lfh::kPathBytes);
         auto deadline = [s](const lfh::Job* j) {
             return j->t_submit + std::min(s->max_offset, (double)j->npix * (double)j->target * s->sec_per_sample);
@@ -869,11 +881,21 @@ int lfh_server_result(lfh_server* s, int64_t id, float* dst, int32_t w, int32_t 
     if (j.state != 2 && j.state != 1) return sfail(s, LFH_E_STATE, "lfh_server_result: job has no samples");
     if (w != j.opt.width || h != j.opt.height) return sfail(s, LFH_E_INVALID, "lfh_server_result: size mismatch");
     const size_t bytes = (size_t)j.npix * 12;
-    if (s->out.bytes < bytes) SCHK(s, s->out.alloc(bytes), "lfh_server_result: alloc");
+    // the image buffer stays for the next result where the budget has room for it
+    // (an allocation and a release per call otherwise); two threads' results take turns
+    DevBuf here;
+    DevBuf* out = &s->out;
+    std::lock_guard<std::mutex> lk(s->mu);
+    if (s->out.bytes < bytes) {
+        drop_image(s);
+        if (s->used + (int64_t)bytes > s->budget) out = &here;
+        SCHK(s, out->alloc(bytes), "lfh_server_result: alloc");
+        s->used += (int64_t)s->out.bytes;
+    }
     SCHK(s, pt_output(j.accum.as<float4>(), j.comp.as<float4>(), j.npix, 1.0f / (float)std::max(1, j.spp_done),
-                      s->out.as<float>(), s->stream),
+                      out->as<float>(), s->stream),
          "lfh_server_result: kernel");
-    SCHK(s, s->readback.read(dst, s->out.p, bytes, nullptr, nullptr, s->device, s->stream),
+    SCHK(s, s->readback.read(dst, out->p, bytes, nullptr, nullptr, s->device, s->stream),
          "lfh_server_result: copy");
     return LFH_OK;
 }

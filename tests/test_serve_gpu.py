@@ -1,6 +1,8 @@
 """Render service: continuous batching of jobs whose rays share the wavefront
 queues.  A job's image is bit-identical alone, in a mix, and through the
 single-scene Renderer surface; admission respects the device budget."""
+import re
+
 import numpy as np
 import pytest
 
@@ -264,3 +266,59 @@ def test_reset_guides_restarts_guided_jobs_from_scratch():
     srv.run_until_idle()
     srv.release(j)
     srv.close()
+
+
+def test_result_image_gives_way_to_jobs_within_the_budget():
+    """The image buffer of lfh_server_result is within the server's budget: on
+    a server that has room for exactly one job, the job after a read result is
+    admitted as before, and no image is held beside it."""
+    import torch
+    print("[serve] result image in the budget", flush=True)
+    w, h = 4000, 3001                     # 144 MB of floats
+    sc = scenes.cornell(w, h, max_depth=2)
+    with pytest.raises(lfh.LfhError) as e:
+        lfh.Server(budget_bytes=1 << 20, max_jobs=2).submit_scene(sc, 1)
+    assert e.value.code == -7
+    need = int(re.search(r"needs (\d+) device bytes", str(e.value)).group(1))
+    srv = lfh.Server(budget_bytes=need, max_jobs=2)
+
+    def render(passes):
+        j = srv.submit_scene(sc, passes)
+        srv.run_until_idle()
+        assert srv.status(j).state == 2
+        return j
+
+    a = render(1)
+    free0 = torch.cuda.mem_get_info()[0]
+    img = srv.result(a, w, h)
+    srv.release(a)
+    b = render(1)
+    free1 = torch.cuda.mem_get_info()[0]
+    assert free0 - free1 < 32 << 20, (free0, free1)
+    assert np.array_equal(srv.result(b, w, h).view(np.uint32), img.view(np.uint32))
+
+
+def test_results_read_by_several_threads_are_each_its_own_job():
+    """Results of different jobs and sizes (below and above the pinned
+    staging's piece) read at once by several threads."""
+    import threading
+    print("[serve] results by threads", flush=True)
+    srv = lfh.Server(max_jobs=8)
+    sizes = [(64, 48), (512, 300), (700, 401), (300, 200)]
+    ids = [srv.submit_scene(scenes.cornell(w, h, max_depth=2), 1 + k) for k, (w, h) in enumerate(sizes)]
+    srv.run_until_idle()
+    want = [srv.result(j, *s) for j, s in zip(ids, sizes)]
+    wrong = []
+
+    def read(k):
+        for _ in range(20):
+            if not np.array_equal(srv.result(ids[k], *sizes[k]), want[k]):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(len(ids))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
+    assert len({w.tobytes() for w in want}) == len(want)
