@@ -339,7 +339,7 @@ int  lfh_path_trace_rays(lfh_ctx* ctx, const float* rays6, uint32_t* seeds, int6
  * forbid hipMalloc).  d_rays6: n x 6 floats (origin, direction); d_seeds: n x 4
  * uint32 pcg4d states (read only); d_radiance: n x 3 floats; all device
  * pointers, asynchronous on the ctx stream.  The path state lives in a static
- * device array of about 19 MiB per GPU (held until the process ends), so n is
+ * device array of about 18 MiB per GPU (held until the process ends), so n is
  * at most 65536 (larger n: LFH_E_INVALID); every call on one GPU shares that
  * array, so calls that overlap on one GPU (other streams or host threads)
  * race.  Radiance is bitwise that of lfh_path_trace_rays. */

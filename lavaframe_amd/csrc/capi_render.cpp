@@ -160,7 +160,7 @@ static int read_output(lfh_ctx* c, void* dst, size_t bytes, const char* fn) {
 }
 
 // Paths per wavefront targeted by multi-sample passes over one-tile frames
-// (292 B of path state each, 9.8 GB at 2^25).  The last bounces of a
+// (284 B of path state each, 9.5 GB at 2^25).  The last bounces of a
 // wavefront hold few paths and cost a traversal's memory latency per launch,
 // so several passes share them.  2^23 -> 2^24: instanced 1080p scene 326 ->
 // 366 Msamples/s; guided / plain time on the guiding room 1.028 / 1.654 s ->

@@ -138,12 +138,15 @@ struct RenderState {
     int64_t npix = 0;
 };
 
+constexpr int64_t kPathBytes = 284;   // device bytes of a PassBufs per path
+
 // Path state + queues of one wavefront pass for up to `cap` paths.
 struct PassBufs {
-    DevBuf rad, thr, absorb, rng, texc, nee;  // per path (nee: 3 float4)
+    // per path 16 B each; nee: 48 B, texc: 8 B, ray and hit queues: 32 B, shadow queue: 64 B, job: 4 B
+    DevBuf rad, thr, absorb, rng, texc, nee;
     DevBuf rq0, rq1, hq, sq;                  // ray queues, hit queue, shadow queue
     DevBuf counters, work;
-    DevBuf job;                               // int per path (multi-job passes)
+    DevBuf job;                               // multi-job passes only
     int cap = 0;
     // All or nothing: on any failure every buffer is released and cap is 0,
     // so the next caller that needs paths allocates again instead of
@@ -174,16 +177,15 @@ private:
     hipError_t alloc_all(int n, hipStream_t s) {
         if (lfh_internal::inject_fault(lfh_internal::kFaultPathAlloc)) return hipErrorOutOfMemory;
         hipError_t e;
-        const size_t f4 = 16;
-        DevBuf* b[10] = {&rad, &thr, &absorb, &rng, &texc, &nee, &rq0, &rq1, &hq, &sq};
-        const size_t m[10] = {1, 1, 1, 1, 1, 3, 2, 2, 2, 4};
-        for (int i = 0; i < 10; ++i)
-            if ((e = b[i]->alloc(f4 * m[i] * (size_t)n)) != hipSuccess) return e;
+        DevBuf* b[11] = {&rad, &thr, &absorb, &rng, &texc, &nee, &rq0, &rq1, &hq, &sq, &job};
+        const size_t m[11] = {16, 16, 16, 16, 8, 48, 32, 32, 32, 64, 4};
+        static_assert(16 * 4 + 8 + 48 + 3 * 32 + 64 + 4 == kPathBytes, "bytes per path");
+        for (int i = 0; i < 11; ++i)
+            if ((e = b[i]->alloc(m[i] * (size_t)n)) != hipSuccess) return e;
         if ((e = counters.alloc(64)) != hipSuccess) return e;
         if ((e = work.alloc(lfhd::kWorkWords * 8)) != hipSuccess) return e;
         if ((e = hipMemsetAsync(counters.p, 0, 64, s)) != hipSuccess) return e;
         if ((e = hipMemsetAsync(work.p, 0, lfhd::kWorkWords * 8, s)) != hipSuccess) return e;
-        if ((e = job.alloc(4 * (size_t)n)) != hipSuccess) return e;
         return hipSuccess;
     }
 };

@@ -24,15 +24,15 @@
 namespace {
 
 constexpr int64_t kNoAllocPaths = (int64_t)1 << 16;   // paths per call, at most
-// per path: rad, thr, absorb, rng, texc (16 B each), nee (48), two ray queues
-// (32 each), hit queue (32), shadow queue (64), job id (4)
+// per path, as in PassBufs: rad, thr, absorb, rng (16 B each), texc (8), nee (48),
+// two ray queues (32 each), hit queue (32), shadow queue (64), job id (4)
 constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 constexpr size_t kF4 = (size_t)kNoAllocPaths * 16;
 constexpr size_t kCountersBytes = 64;
 constexpr size_t kWorkBytes = align_up((size_t)lfhd::kWorkWords * 8);
-constexpr size_t kScratchBytes = kF4 * (5 + 3 + 2 + 2 + 2 + 4) + align_up((size_t)kNoAllocPaths * 4) +
-                                 kCountersBytes * 4 + kWorkBytes;   // 18.9 MiB
+constexpr size_t kScratchBytes = (size_t)kNoAllocPaths * lfh::kPathBytes + kCountersBytes * 4 + kWorkBytes;   // 17.8 MiB
+static_assert((size_t)kNoAllocPaths * 4 % kAlign == 0, "every array ends on a boundary of kAlign");
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -99,7 +99,7 @@ extern "C" int lfh_path_trace_rays_device_noalloc(lfh_ctx* c, const float* d_ray
     pb.thr = reinterpret_cast<float4*>(take(kF4));
     pb.absorb = reinterpret_cast<float4*>(take(kF4));
     pb.rng = reinterpret_cast<uint4*>(take(kF4));
-    pb.texc = reinterpret_cast<float2*>(take(kF4));
+    pb.texc = reinterpret_cast<float2*>(take(kF4 / 2));
     pb.nee = reinterpret_cast<float4*>(take(3 * kF4));
     pb.stride = kNoAllocPaths;
     PtQueues q;

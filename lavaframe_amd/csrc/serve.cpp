@@ -47,8 +47,6 @@ namespace lfh {
 
 namespace {
 
-// Device bytes of one pass's path state + queues per path (PassBufs).
-constexpr int64_t kPathBytes = 16 * (1 + 1 + 1 + 1 + 1 + 3 + 2 + 2 + 2 + 4) + 4;
 constexpr int64_t kAccumBytes = 32;  // sum + compensation, float4 each
 #ifndef LFH_SERVE_GUIDE_LR
 // Adam learning rate of a served scene's guide.  Guiding room on one warm server, median

@@ -322,3 +322,14 @@ def test_results_read_by_several_threads_are_each_its_own_job():
         t.join()
     assert wrong == []
     assert len({w.tobytes() for w in want}) == len(want)
+
+
+def test_a_job_is_charged_what_its_paths_and_images_take():
+    """32 B of accumulation and 284 B of path state per pixel, beside its scene."""
+    print("[serve] bytes of a job", flush=True)
+    need = []
+    for w, h in ((64, 64), (192, 64)):
+        with pytest.raises(lfh.LfhError) as e:
+            lfh.Server(budget_bytes=1000, max_jobs=1).submit_scene(scenes.cornell(w, h), 1)
+        need.append(int(re.search(r"needs (\d+) device bytes", str(e.value)).group(1)))
+    assert need[1] - need[0] == 128 * 64 * (32 + 284)
