@@ -79,17 +79,33 @@ struct LaneStack {
 // 64 / 128 / 192 / 256: 16.8M-ray closest hit 5.95 / 5.59 / 5.44 / 5.41 ms, 2M-ray any hit 765 / 749 / 781 / 787 us,
 // 8.4M incoherent rays 3.50 / 3.52 / 3.57 / 3.58 ms, C0 2.41 / 2.31 / 2.33 / 2.32 ms, viewer 720p 9.52 / 9.31 / 9.42 /
 // 9.52 ms, served mix 4.68 / 4.56 / 4.61 / 4.65 ms: longer chunks save atomics, and leave the waves that end a queue
-// with more rays each
+// with more rays each.
+// The length is also the line between queues that are all owned and queues with dynamic fetches (closest hit: 328k
+// rays at 64, 655k at 128; any hit 393k and 786k).  Batches of incoherent / pinhole rays, 1M triangles, closest hit,
+// 64 against 128:
+//   300k          293 / 196 us against 293 / 206    both lengths all owned
+//   400k          361 / 275 against 340 / 252       between the lines
+//   650k          472 / 323 against 437 / 339
+//   780k          508 / 369 against 569 / 418       just past the longer line: few waves end with a chunk more
+//   1.3M          725 / 487 against 724 / 501
+//   2M            986 / 653 against 1012 / 680
+//   from 3.2M on  equal to 1 %
+// Any hit 0.95-1.10 times its time with 128 between the lines, 0.92-1.05 up to 2M.  128 for all, because the
+// path tracer's queues prefer it at every depth (64: C0 2.37 against 2.27 ms, viewer 9.70 against 9.28, and 2 %
+// longer in both with 64 only for queues of one to four times the line).
 #define LFH_FETCH_CHUNK 128
 #endif
 #ifndef LFH_FETCH_MIN
-// 1021 rays, 20k triangles: at least 1 / 4 / 16 / 64 rays per wave 71 / 97 / 115 / 110 us (159 us with
-// every wave asking all eight counters); textured 128 x 128 tiles 234 / 239 / 240 / 241 us per pass (738)
+// at least 1 / 4 / 16 rays per wave, closest hit, 1M triangles: 1k incoherent rays 93 / 123 / 137 us, 5k 118 / 128 /
+// 155, 20k 179 / 179 / 187, 50k 195 / 195 / 189; 20k triangles, pinhole: 1k 57 / 73 / 74, 20k 71 / 71 / 61, 50k 88 / 88 /
+// 73 (coherent rays of a wave cost little more than one).  A pick of 1021 rays 67 / 77 / 92 us, textured 128 x 128
+// tiles 172 / 165 / 164 us per pass, viewer 9.28 / 9.24 / 9.37 ms: 1 for the smallest calls.
 #define LFH_FETCH_MIN 1
 #endif
 #ifndef LFH_FETCH_OWNED
-// eighths of a large queue owned by position: 0 / 4: C0 3.34 / 3.29 ms, 16.8M-ray closest hit 10.32 / 10.23 ms
-// (6: longer when half of the slices hold cheap rays, since owned chunks are never passed on)
+// eighths of a large queue owned by position: 0 / 4 / 6: viewer 9.36 / 9.22 / 9.30 ms, C0 2.27 / 2.27 / 2.28; batches of
+// 0.9M-8.4M rays the same with 0, 2 and 4, and up to 6 % longer with 6 (8.4M pinhole rays, 20k triangles 1.53 ->
+// 1.62 ms: owned chunks are never passed on)
 #define LFH_FETCH_OWNED 4
 #endif
 constexpr int kFetchChunk = LFH_FETCH_CHUNK;
