@@ -3,6 +3,8 @@ changes: one ray, fewer rays than waves, exactly the rays the launch's waves
 own by position, one more, and a second owned round.  Every ray of a batch is
 traced exactly once, so the hits of any split equal those of the CPU oracle
 bit for bit (ids and the bits of t, u, v)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -11,29 +13,51 @@ from oracle import native
 
 pytestmark = pytest.mark.gpu
 
-# 256 CUs x 5 or 6 blocks x 4 waves x 128 rays: the largest queues without dynamic fetches
-CLOSEST, ANY = 256 * 5 * 4 * 128, 256 * 6 * 4 * 128
+CHUNK = int(re.search(r"#define LFH_FETCH_CHUNK (\d+)",
+                      (lfh.PKG_DIR / "csrc" / "dev_trace.h").read_text()).group(1))
+WAVES = 4          # per block
 
 
 @pytest.fixture(scope="module")
 def world():
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
     sc = scenes.soup(300, seed=3)
-    rays = scenes.incoherent_rays(4 * ANY + 77, seed=4)
-    return lfh.Context.from_scene(sc), native.OracleScene(sc.arrays()), rays
+    # rays that one block per CU owns without dynamic fetches; a kernel's occupancy is 1 to 8 blocks
+    line = cus * WAVES * CHUNK
+    rays = scenes.incoherent_rays(33 * line + 77, seed=4)
+    orc = native.OracleScene(sc.arrays())
+    return lfh.Context.from_scene(sc), orc.trace_closest(rays), orc.trace_any(rays), rays, line
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 5119, 5121, 65537, CLOSEST - 1, CLOSEST, CLOSEST + 1, ANY - 1, ANY + 1,
-                               2 * CLOSEST + 63, 4 * ANY + 77])
-def test_every_ray_of_a_batch_is_traced_once(world, n):
+def _check(world, n):
     print(f"[fetch] {n} rays", flush=True)
-    ctx, orc, rays = world
+    ctx, hits, occ, rays, _ = world
     r = rays[-n:]
-    got, want = ctx.trace_closest(r), orc.trace_closest(r)
+    got, want = ctx.trace_closest(r), hits[-n:]
     for f in ("prim", "inst", "mat"):
         assert np.array_equal(got[f], want[f]), f
     for f in ("t", "u", "v"):
         assert np.array_equal(got[f].view(np.uint32), want[f].view(np.uint32)), f
-    assert np.array_equal(ctx.trace_any(r), orc.trace_any(r))
+    assert np.array_equal(ctx.trace_any(r), occ[-n:])
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 5119, 5121, 65537])
+def test_every_ray_of_a_small_batch_is_traced_once(world, n):
+    _check(world, n)
+
+
+@pytest.mark.parametrize("blocks", range(1, 9))
+@pytest.mark.parametrize("past", [-1, 0, 1])
+def test_every_ray_is_traced_once_around_the_owned_share(world, blocks, past):
+    """Every occupancy that a traversal kernel can have, so whatever its
+    register count, one of them is the boundary of each kernel."""
+    _check(world, blocks * world[4] + past)
+
+
+@pytest.mark.parametrize("lines", [9, 12, 33])   # 33: a second owned round at any occupancy
+def test_every_ray_of_a_large_batch_is_traced_once(world, lines):
+    _check(world, lines * world[4] + 63)
 
 
 @pytest.mark.parametrize("ntri", [4, 1000, 30000])
