@@ -321,6 +321,25 @@ def test_batched_passes_equal_sequential_passes():
     assert sa.sum() > 0
 
 
+@pytest.mark.parametrize("passes", [1, 2, 3, 4, 5, 7, 9])
+def test_batches_of_any_length_are_added_in_order(passes):
+    """Accumulation takes four samples of a pixel at a time: batches below,
+    at and past a multiple of four add the same sums, bit for bit, as the
+    passes one by one."""
+    print(f"[pt] batch of {passes}", flush=True)
+    sc = scenes.cornell(37, 19)
+    cam = sc.camera()
+    a, b = ctx_of(sc), ctx_of(sc)
+    a.update(cam, reset=True)
+    a.render_passes(passes)
+    b.update(cam, reset=True)
+    for _ in range(passes):
+        b.update(cam)
+        b.render()
+    for x, y in zip(a.accum(), b.accum()):
+        np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
+
+
 def _sphere_light(center, radius, emission):
     area = np.float32(4.0 * math.pi * radius * radius)
     return np.concatenate([np.asarray(center, np.float32), np.asarray(emission, np.float32), np.zeros(6, np.float32),
