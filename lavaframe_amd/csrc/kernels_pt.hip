@@ -693,9 +693,11 @@ __global__ __launch_bounds__(256) void k_accumulate(PathBufs pb, int total, CamP
     const int nb = cam.batch > 1 ? cam.batch : 1;
     const int P = cam.tile_w * cam.tile_h;
     // Bound by the chain of a thread's own loads where pixels are few (256 x 256 at 64 samples is one wave per
-    // SIMD, 94 % of its time waiting), so four samples' loads are in flight together (C0 frame 2.30 -> 2.27 ms;
-    // frames with more pixels the same).
-    constexpr int kAhead = 4;
+    // SIMD, 94 % of its time waiting), so four samples' loads are in flight together: 73 -> 54 us, C0 frame 2.30 ->
+    // 2.27 ms, 1080p the same.  That takes 84 VGPRs, 5 waves per SIMD instead of 8, which costs more than it gives
+    // where pixels are many: 18 passes of a served 720p frame 146 -> 163 us.  A server's wavefronts hold the pixels
+    // of all its jobs, so they take one sample at a time.
+    constexpr int kAhead = MULTI ? 1 : 4;
     for (int k0 = 0; k0 < nb; k0 += kAhead) {
         const int m = nb - k0 < kAhead ? nb - k0 : kAhead;
         float4 r4[kAhead];
