@@ -63,7 +63,7 @@ LFH_HD uint32_t make_inst(uint32_t inst) { return kRefInstBit | inst; }
 #define LFH_TRACE_WAVES 5
 #endif
 #ifndef LFH_ANYHIT_WAVES
-// the same for any hit (79 VGPRs): 5 and 6 waves 0.794 ms for 2.1M rays
+// the same for any hit (80 VGPRs): 5 and 6 waves 0.794 ms for 2.1M rays
 #define LFH_ANYHIT_WAVES 6
 #endif
 // Work counters of the persistent traversal kernels: a queue's ray ids are

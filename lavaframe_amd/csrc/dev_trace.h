@@ -344,12 +344,14 @@ LFH_DEV void load_node(const TraceScene& sc, const TraceState& s, uint32_t cur, 
 // BVH4 node: slab-test the four child boxes, push the hit children last in
 // order first.  Returns the first one, or kRefSentinel when none is hit.
 //
-// Bound by VALU issue (82 % busy on 16.8M mixed rays, 40 % of the lanes active
-// on average): the test is 17 instructions per child, the sort 25, the pushes
+// Bound by VALU issue (83 % busy on 16.8M mixed rays, 40 % of the lanes active
+// on average) and close behind it by node traffic: 43 % of the requests hit L2,
+// and the rest moves 22.9 GB per launch at 4.1-4.2 TB/s, 86 % of what a copy
+// reaches.  The test is 17 instructions per child, the sort 25, the pushes
 // 12 without a branch per child.  With one pop per step for all lanes and the
 // order keys of slab_entry the 1M-triangle soup's closest hit went from 1650 to
 // 2840 Mrays/s (incoherent half 1037 -> 2380), any hit from 3270 to 3960;
-// with 128-ray reservations they are 3050 and 4840.
+// with 128-ray reservations they are 3010-3070 and 4720-4850.
 // Loading the nodes of a step before its leaf tests, to overlap the two
 // latencies, spills (6.24 against 5.95 ms; any hit 6.9 against 2.2 ms).
 template <bool ANY, bool STATS>

@@ -6,10 +6,10 @@
 //   A (16 x 32):  row l%16, k = (l/16)*8 .. +7     (8 BF16 = 16 B per lane)
 //   B (32 x 16):  col l%16, k = (l/16)*8 .. +7
 //   D (16 x 16):  col l%16, rows (l/16)*4 .. +3    (4 FP32)
-// Training: activations live in LDS as BF16 rows of kPitch elements (64 + 8
-// padding so that the 16 B fragment reads of 16 consecutive rows spread over
-// the banks); weights are read as B fragments straight from global memory
-// (32 KiB per direction, resident in L1/L2).  Inference: the encoded inputs
+// Training: activations, gradients and the current product's weights live in LDS
+// as BF16 rows of kPitch elements (64 + 8 padding so that the 16 B fragment
+// reads of 16 consecutive rows spread over the banks); the weights are fetched
+// one product ahead.  Inference: the encoded inputs
 // pass through LDS once, then the MLP runs transposed with the weights held in
 // registers and the activations never leaving their lanes (k_guide_infer).
 #include <algorithm>

@@ -3,11 +3,14 @@
 // One TiledRenderer pass over a tile (renderer.glsl:main + PathTrace,
 // pathtrace.glsl:208-295) is split into stages that pass SoA queues through
 // HBM:
-//   generate  camera rays for the tile pixels, path state init
-//   extend    closest hit (analytic lights first, then the BVH) per queued ray
+//   generate  camera rays for the tile pixels and the paths' random-number state;
+//             shading of depth 0 starts the rest of the path state
+//   extend    closest hit (analytic lights first, then the BVH) per queued ray;
+//             one launch per depth takes these and the shadow rays of the depth before
 //   shade     miss / emitter / surface shading, next-event candidates, BSDF
 //             sampling, Russian roulette; appends continuing rays and shadow
-//             rays with one atomic per block (ballot + rank, block offsets in LDS)
+//             rays with one atomic per block (ballot + rank, block offsets in LDS);
+//             folds in the next-event terms of the depth before
 //   shadow    any hit per shadow ray; clears the candidate when occluded
 //   accumulate  pending next-event terms + Kahan-compensated accumulation
 // The random-number stream of each path is the reference's: it lives in the
